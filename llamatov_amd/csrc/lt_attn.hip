@@ -1551,6 +1551,15 @@ bool use_rm() {
   return on;
 }
 
+// LT_ATTN_MM=0 keeps prefill on the per-row kernels (for comparisons).
+bool use_mm() {
+  static const bool on = [] {
+    const char* s = getenv("LT_ATTN_MM");
+    return !(s && s[0] == '0');
+  }();
+  return on;
+}
+
 // LT_ATTN_W1=0 keeps every mode on k_attn (for comparisons); the default is k_attn_w1
 // wherever its head sizes and LDS budget apply.
 bool use_w1() {
@@ -1609,12 +1618,24 @@ int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, 
   // fp16: 64, 128 or 256 dims; fp32: 64 or 128 (a K row of 8 to 32 16-byte units)
   const bool w1 = use_w1() && A.hd % 64 == 0 &&
                   (f16 ? (dpl == 1 || dpl == 2 || dpl == 4) : (dpl == 1 || dpl == 2)) && w1_shm <= 64 * 1024;
+  // prefill on the matrix cores, for what the per-row kernels take too (their LDS limits and the
+  // workspace the caller owes a split context stand)
+  const bool mm = mode == AM_PREFILL && use_mm() && lt_attn_mm_covers(A.hd, rows, A.maxt, A.nsplit) &&
+                  (w1 || ((size_t)hpw * A.hd + 2 * A.hd + (size_t)hpw * per_max + kVChunkFloats) * sizeof(float) <=
+                             64 * 1024);
+  auto launch_mm = [&]() {
+    LtAttnMm M = {};
+    M.q = A.q; M.q_stride = A.q_stride; M.kc = A.kc; M.vc = A.vc; M.len = A.len; M.out = A.out;
+    M.T = rows; M.nh = A.nh; M.nkv = A.nkv; M.scale = A.scale; M.maxt = A.maxt; M.nsplit = A.nsplit;
+    return lt_attn_mm_prefill(ctx, M, A.hd, f16);
+  };
   // a prefill row's splits in one wave (AM_PREFILL_RM): at most 64 positions per split (each
   // lane of a split's Z tree then holds one position) and the whole row's scores in LDS
   const size_t per_up_rm = (size_t)(A.maxt + ring - 1) / ring * ring;
   const size_t rm_shm = ((size_t)h * A.hd + kpr * (ku + 1) * 4 + ((per_up_rm + 8 + 1 + 64) * h + 3) / 4 * 4 +
                          3 * (size_t)A.nsplit * h + h) * sizeof(float);
   if (w1 && mode == AM_PREFILL && A.nsplit > 1 && per_max <= 64 && rm_shm <= 64 * 1024 && use_rm()) {
+    if (mm) return launch_mm();
     A.per_max = A.maxt;
     const dim3 grid(1, A.nh / h, rows);
     const hipError_t e = f16 ? launch_w1<true, AM_PREFILL_RM>(h, dpl, grid, rm_shm, ctx->stream, A)
@@ -1633,6 +1654,7 @@ int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, 
     A.wsz = w.z;
     A.wso = w.o;
   }
+  if (mm) return launch_mm();
   // decode with 2, 4, 7 or 8 query heads per KV group on a grid of at most 4 workgroups per CU
   // (batch 1): one wave per head, K and V staged once per workgroup through LDS.  On larger
   // grids its LDS footprint (3 workgroups per CU at 16k) loses to the single-wave kernel's

@@ -67,6 +67,25 @@ static inline AttnWs lt_attn_ws_layout(void* ws, int rows, int hd, int nsplit) {
   return w;
 }
 
+// Causal prefill attention on the matrix cores (lt_attn_mm.hip): T query rows (q_stride floats
+// apart) of one sequence over its cache, query t attending *len + t + 1 positions.
+struct LtAttnMm {
+  const float* q;
+  int q_stride;
+  const void* kc;
+  const void* vc;
+  const int* len;
+  float* out;
+  int T, nh, nkv;
+  float scale;
+  int maxt, nsplit;
+  int cap, ntiles;   // set by the launcher: positions held in LDS, 16-row tiles in the grid
+};
+// Head sizes 64 and 128; one split, or a multiple of 16 splits over a long prompt whose context
+// fits in LDS.
+bool lt_attn_mm_covers(int hd, int T, int maxt, int nsplit);
+int lt_attn_mm_prefill(lt_ctx* ctx, LtAttnMm A, int hd, bool f16);
+
 // Device helpers shared by the kernel translation units.
 __device__ __forceinline__ float lt_h2f(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));

@@ -132,6 +132,44 @@ __device__ __forceinline__ float wave_max(float a) {
   return halfwave_max(a);
 }
 
+// lt_expf_sel of N values at once, written stage by stage so that the N binary64 chains
+// interleave, and held straight-line: the compiler otherwise turns lt_expf_sel's selects into
+// branches around its polynomial and runs one value after the other (attention's softmax, four
+// values a lane: 1470 -> 700 cycles).  Equal to lt_expf_sel for every input (a nan is clamped
+// to -120 here and put back by the last select).
+template <int N>
+__device__ __forceinline__ void lt_expf_n(float (&x)[N]) {
+  double r[N], k[N], p[N];
+  float v[N];
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    r[i] = (double)fminf(fmaxf(x[i], -120.0f), 100.0f);
+    k[i] = __builtin_rint(r[i] * LT_LOG2E);
+  }
+#pragma unroll
+  for (int i = 0; i < N; i++) r[i] = fma(-k[i], LT_LN2_HI, r[i]);
+#pragma unroll
+  for (int i = 0; i < N; i++) r[i] = fma(-k[i], LT_LN2_LO, r[i]);
+  constexpr double c[12] = {1.0 / 39916800.0, 1.0 / 3628800.0, 1.0 / 362880.0, 1.0 / 40320.0, 1.0 / 5040.0, 1.0 / 720.0,
+                            1.0 / 120.0,      1.0 / 24.0,      1.0 / 6.0,      0.5,           1.0,          1.0};
+#pragma unroll
+  for (int i = 0; i < N; i++) p[i] = 1.0 / 479001600.0;
+#pragma unroll
+  for (int j = 0; j < 12; j++)
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = fma(p[i], r[i], c[j]);
+#pragma unroll
+  for (int i = 0; i < N; i++) v[i] = (float)(p[i] * lt_u2d((uint64_t)((int)k[i] + 1023) << 52));
+#pragma unroll
+  for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    v[i] = x[i] > 100.0f ? __builtin_inff() : v[i];
+    v[i] = x[i] < -120.0f ? 0.0f : v[i];
+    x[i] = x[i] != x[i] ? x[i] : v[i];
+  }
+}
+
 // ---- the engine quantizer without per-element division -----------------------------
 // d16 = fp16(amax/127) (1 if not amax > 0) by the hardware conversion v_cvt_f16_f32
 // (round to nearest even, gradual underflow, overflow to inf: the bits of
