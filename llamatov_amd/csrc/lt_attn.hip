@@ -68,16 +68,6 @@ struct AttnArgs {
 
 constexpr int kMaxInWgSplits = 16;   // splits one workgroup can hold (partial outputs in registers)
 
-// Where block g of the quantized output goes (g counts the blocks of the [rows][nh*hd] output
-// row by row): row-major, or with obm > 0 block-major over obm rows -- quants [nh*hd/32][obm]
-// [32], scales [nh*hd/32][obm], the tiled GEMM's activation layout.
-__device__ __forceinline__ size_t q8_out_block(int obm, int nh, int hd, size_t g) {
-  if (obm <= 0) return g;
-  const size_t nbr = (size_t)(nh * hd / 32);
-  const size_t row = g / nbr;
-  return (g - row * nbr) * (size_t)obm + row;
-}
-
 template <bool kF16>
 __device__ __forceinline__ float kv_round(float v) {
   return kF16 ? lt_half_to_float_bits(lt_float_to_half_bits(v)) : v;
@@ -1560,6 +1550,15 @@ bool use_mm() {
   return on;
 }
 
+// LT_ATTN_HEAD=0 keeps unsplit decode attention on the kernels below (for comparisons).
+bool use_head() {
+  static const bool on = [] {
+    const char* s = getenv("LT_ATTN_HEAD");
+    return !(s && s[0] == '0');
+  }();
+  return on;
+}
+
 // LT_ATTN_W1=0 keeps every mode on k_attn (for comparisons); the default is k_attn_w1
 // wherever its head sizes and LDS budget apply.
 bool use_w1() {
@@ -1655,6 +1654,15 @@ int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, 
     A.wso = w.o;
   }
   if (mm) return launch_mm();
+  if ((mode == AM_STEP || mode == AM_DECODE) && A.nsplit == 1 && use_head() &&
+      (w1 || ((size_t)hpw * A.hd + 2 * A.hd + (size_t)hpw * per_max + kVChunkFloats) * sizeof(float) <= 64 * 1024) &&
+      lt_attn_head_covers(ctx, rows, A.nh, A.hd, A.maxt)) {
+    LtAttnHead H = {};
+    H.qkv = A.qkv; H.freqs = A.freqs; H.q = A.q; H.q_stride = A.q_stride; H.kc = A.kc; H.vc = A.vc; H.len = A.len;
+    H.out = A.out; H.oq = A.oq; H.od = A.od; H.obm = A.obm; H.batch = rows; H.nh = A.nh; H.nkv = A.nkv;
+    H.scale = A.scale; H.maxt = A.maxt;
+    return lt_attn_head(ctx, H, A.hd, f16, mode == AM_STEP);
+  }
   // decode with 2, 4, 7 or 8 query heads per KV group on a grid of at most 4 workgroups per CU
   // (batch 1): one wave per head, K and V staged once per workgroup through LDS.  On larger
   // grids its LDS footprint (3 workgroups per CU at 16k) loses to the single-wave kernel's

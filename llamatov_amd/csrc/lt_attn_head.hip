@@ -1,0 +1,322 @@
+// lt_attn_head.hip -- decode attention of one query head over one sequence's cache, unsplit (the
+// single-pass order of k_attn_decode_masked): the decode step (RoPE, KV append, attention,
+// quant) and batched decode, bit-identical to k_attn_w1 and k_attn_dec of lt_attn.hip.
+//
+// The unsplit order leaves one serial chain per (head, dim) over all positions, so a head's
+// latency is what counts: a workgroup of NW waves takes one head and shares out everything that
+// is not that chain.
+//   scores   rounds of 64 positions, a wave every NW-th: rows come in by whole 128-byte lines,
+//            pass through the wave's own LDS (padded) and lane l runs position l's chain;
+//   softmax  the exps over all threads, Z by one wave (64-lane fold and tree);
+//   O        on the fp32 matrix cores, whose v_mfma_f32_16x16x4_f32 is a sequential fma chain
+//            over its four products (lt_attn_mm.hip): 16 DT dims a wave, four positions an
+//            instruction, the exps broadcast to all 16 columns.  One instruction per 32 cycles
+//            for four positions beats four dependent vector fmas with their operand reads; the
+//            operands are read from LDS a block ahead.
+// K rows are requested before the length is known; V rows past it are replaced by zeros.
+//
+// The heads of a KV group run on one XCD (workgroups are dealt to the 8 XCDs round-robin), so a
+// group's rows are fetched into one L2 once.
+#include "lt_q8_device.h"
+
+namespace {
+
+using namespace lt;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Position t's slot in the exps: a lane of group k reads its four steps' exps (t = 4 i + k, i =
+// 0..3) of a 16-position tile as one 16-byte word.
+__device__ __forceinline__ int e_slot(int t) { return (t & ~15) | ((t & 3) << 2) | ((t >> 2) & 3); }
+
+template <bool kF16, int HD, int NW, bool kStep>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 2))) void k_attn_head(
+    LtAttnHead A) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  constexpr int kEb = kF16 ? 2 : 4;
+  constexpr int NL = HD * kEb / 128;                // 128-byte lines per cache row
+  constexpr int R = NL == 1 ? 2 : 4;                // K lines (of 64 rows) in flight
+  constexpr int kKRow = 144;                        // a line's pitch in LDS (lanes 36 banks apart)
+  constexpr int NP = NW < HD / 16 ? NW : HD / 16;   // waves that fold O
+  constexpr int DT = HD / 16 / NP;                  // adjacent dims per lane in O
+  constexpr int kVB = DT * kEb;
+  constexpr int SB = 16 * kVB;                      // a wave's bytes of one V row
+  constexpr int RB = 1024 / SB;                     // V rows per block (one 16-byte load per lane)
+  constexpr int D = 256 / RB;                       // V blocks in flight: 256 rows
+  float* sq = lds;                                  // [HD] q (roped in a step)
+  float* sk = sq + HD;                              // [HD] step: the new k in the cache's format
+  float* sv = sk + HD;                              // [HD] step: the new v through the cache's type
+  float* so = sv + HD;                              // [HD] the output
+  float* sm = so + HD;                              // [NW] maxima, then [1] Z
+  uint8_t* vbuf = (uint8_t*)(sm + 12);              // [NP][2][1024]
+  uint8_t* kbuf = vbuf + NP * 2048;                 // [NW][64][kKRow] K lines
+  float* P = (float*)(kbuf + NW * 64 * kKRow);      // [cap] exps by e_slot
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+  const int n16 = l & 15, g4 = l >> 4;
+
+  const int rep = A.nh / A.nkv;
+  const int slot = (int)blockIdx.x >> 3;
+  const int pair = slot / rep * 8 + ((int)blockIdx.x & 7);    // (sequence, KV group)
+  if (pair >= A.batch * A.nkv) return;
+  const int b = pair / A.nkv, g = pair - b * A.nkv, r0 = slot % rep, h = g * rep + r0;
+
+  const int len0 = A.len[kStep ? 0 : b];
+  const uint32_t pitch = (uint32_t)A.nkv * HD * kEb;
+  const uint32_t seq = (uint32_t)b * (uint32_t)A.maxt * pitch;
+  const uint32_t gb = seq + (uint32_t)g * HD * kEb;
+  const int cache_end = (int)(seq + (uint32_t)A.maxt * pitch);
+  const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc(A.kc, 0, cache_end, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc(A.vc, 0, cache_end, 0x00020000);
+
+  // K line u (line u % NL of round w + NW (u / NL)): row 8 i + l / 8, bytes 16 (l % 8) of the line;
+  // rows past the cache read zeros
+  const uint32_t kb0 = gb + (uint32_t)(l >> 3) * pitch + (uint32_t)(l & 7) * 16u;
+  auto load_k = [&](int u, u32x4 (&k)[8]) {
+    const uint32_t off = kb0 + (uint32_t)((w + NW * (u / NL)) * 64) * pitch + (uint32_t)(u % NL) * 128u;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      k[i] = __builtin_amdgcn_raw_buffer_load_b128(krsrc, (int)(off + (uint32_t)(8 * i) * pitch), 0, 0);
+  };
+  u32x4 kr[R][8];
+#pragma unroll
+  for (int u = 0; u < NL; u++) load_k(u, kr[u]);    // (the first round, before the length)
+  // V block at row p: 16 bytes of row p + l / (SB / 16) per lane
+  const int db = w * 16 * DT;
+  const int vrow = l / (SB / 16);
+  const uint32_t vb = gb + (uint32_t)db * kEb + (uint32_t)(l % (SB / 16)) * 16u;
+  auto load_v = [&](int p) {
+    return __builtin_amdgcn_raw_buffer_load_b128(vrsrc, (int)((uint32_t)(p + vrow) * pitch + vb), 0, 0);
+  };
+
+  int Lnew = -1, n;
+  bool valid = true;
+  if (kStep) {
+    valid = len0 >= 0 && len0 < A.maxt;
+    Lnew = valid ? len0 : -1;
+    n = valid ? len0 + 1 : 0;
+  } else {
+    n = len0 < 0 ? 0 : (len0 > A.maxt ? A.maxt : len0);
+  }
+  const int nv = kStep && valid ? len0 : n;         // rows that come from the cache
+  const int nr = (n + 63) >> 6;
+  const int nu = w < nr ? (nr - w + NW - 1) / NW * NL : 0;   // this wave's K lines
+#pragma unroll
+  for (int u = NL; u < R; u++)
+    if (u < nu) load_k(u, kr[u]);
+  if (kStep) {
+    // RoPE (the arithmetic of k_rope, rope_from_facts.pl:40-69) of q on wave 0 and of the group's
+    // k on wave 1; v on wave 2; k and v through the cache's type
+    auto round_kv = [&](float x) { return kF16 ? lt_half_to_float_bits(lt_float_to_half_bits(x)) : x; };
+    if (w < 2) {
+      const float* src = w == 0 ? A.qkv + (size_t)h * HD : A.qkv + (size_t)A.nh * HD + (size_t)g * HD;
+      if (l < HD / 2) {
+        const float x1 = src[l], x2 = src[l + HD / 2];
+        float sn, cs;
+        lt_sincosf((float)(valid ? len0 : 0) * A.freqs[l], &sn, &cs);
+        const float o1 = fmaf(x1, cs, -(x2 * sn)), o2 = fmaf(x1, sn, x2 * cs);
+        if (w == 1 && kF16) {
+          ((uint16_t*)sk)[l] = lt_float_to_half_bits(o1);
+          ((uint16_t*)sk)[l + HD / 2] = lt_float_to_half_bits(o2);
+        } else {
+          float* dst = w == 0 ? sq : sk;
+          dst[l] = o1;
+          dst[l + HD / 2] = o2;
+        }
+      }
+    } else if (w == 2) {
+#pragma unroll
+      for (int i = 0; i < HD / 64; i++)
+        sv[l + 64 * i] = round_kv(A.qkv[(size_t)(A.nh + A.nkv) * HD + (size_t)g * HD + l + 64 * i]);
+    }
+  } else if (tid < HD) {
+    sq[tid] = A.q[(size_t)b * A.q_stride + (size_t)h * HD + tid];
+  }
+  __syncthreads();
+  if (kStep && valid && r0 == 0 && w == NW - 1) {
+    // the new row into the cache (k_append_kv_incr, dev_residency.py:303-315)
+    const size_t e0 = (size_t)len0 * A.nkv * HD + (size_t)g * HD;
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++) {
+      const int d = l + 64 * i;
+      if (kF16) {
+        ((uint16_t*)A.kc)[e0 + d] = ((const uint16_t*)sk)[d];
+        ((uint16_t*)A.vc)[e0 + d] = lt_float_to_half_bits(sv[d]);
+      } else {
+        ((float*)A.kc)[e0 + d] = sk[d];
+        ((float*)A.vc)[e0 + d] = sv[d];
+      }
+    }
+  }
+
+  // scores
+  uint8_t* const kw = kbuf + w * 64 * kKRow;
+  float mx = -1e30f, acc = 0.0f;
+  for (int u0 = 0; u0 < nu; u0 += R) {
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int u = u0 + i;
+      if (u >= nu) break;
+      const int t0 = (w + NW * (u / NL)) * 64, ln = u % NL;
+#pragma unroll
+      for (int j = 0; j < 8; j++) *(u32x4*)(kw + (8 * j + (l >> 3)) * kKRow + (l & 7) * 16) = kr[i][j];
+      load_k(u + R, kr[i]);
+      if (kStep && Lnew >= t0 && Lnew < t0 + 64 && l < 8)   // the new row over its place
+        *(u32x4*)(kw + (Lnew - t0) * kKRow + l * 16) = *(const u32x4*)((const uint8_t*)sk + ln * 128 + l * 16);
+      asm volatile("" ::: "memory");
+      if (NL == 1 || ln == 0) acc = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 8; c++) {
+        const u32x4 k = *(const u32x4*)(kw + l * kKRow + c * 16);
+        const float* qc = sq + ln * (128 / kEb) + c * (16 / kEb);
+        const uint32_t y[4] = {k.x, k.y, k.z, k.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if (kF16) {
+            acc = fmaf(qc[2 * e], lt_h2f((uint16_t)(y[e] & 0xFFFFu)), acc);
+            acc = fmaf(qc[2 * e + 1], lt_h2f((uint16_t)(y[e] >> 16)), acc);
+          } else {
+            acc = fmaf(qc[e], __uint_as_float(y[e]), acc);
+          }
+        }
+      }
+      if ((NL == 1 || ln == NL - 1) && t0 + l < n) {
+        const float x = acc * A.scale;
+        P[e_slot(t0 + l)] = x;
+        mx = fmaxf(mx, x);
+      }
+    }
+  }
+  u32x4 vr[D];                                      // (under the softmax)
+  if (w < NP) {
+#pragma unroll
+    for (int j = 0; j < D; j++)
+      if (j < 2 || j * RB < nv) vr[j] = load_v(j * RB);
+  }
+  mx = wave_max(mx);
+  if (l == 0) sm[w] = mx;
+  __syncthreads();
+  float m = -1e30f;
+#pragma unroll
+  for (int i = 0; i < NW; i++) m = fmaxf(m, sm[i]);
+  // the exps; zeros up to whole groups of the O loop
+  const int n_up = (nv + D * RB - 1) / (D * RB) * (D * RB);
+  const int n_all = n_up > n ? n_up : n;
+  for (int t = tid; t < n_all; t += 128 * NW) {
+    const int t1 = t + 64 * NW;
+    float e[2];
+    e[0] = P[e_slot(t)] - m;
+    e[1] = P[e_slot(t1 < n_all ? t1 : t)] - m;
+    lt_expf_n(e);
+    P[e_slot(t)] = t < n ? e[0] : 0.0f;
+    if (t1 < n_all) P[e_slot(t1)] = t1 < n ? e[1] : 0.0f;
+  }
+  __syncthreads();
+  if (w == NW - 1) {
+    float z = 0.0f;
+    for (int t = l; t < n; t += 64) z = z + P[e_slot(t)];
+    z = wave_tree_dpp(z);
+    if (l == 0) sm[NW] = z;
+  }
+
+  // O: the cached rows in ascending order; a step's new row, the last, from LDS
+  f32x4 o[DT];
+#pragma unroll
+  for (int d = 0; d < DT; d++) o[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (w < NP) {
+    uint8_t* const vw = vbuf + w * 2048;
+    auto put_v = [&](int buf, u32x4 x, int p) {
+      if (p + RB > nv) {                            // rows past the length may hold anything
+        const bool in = p + vrow < nv;
+        x = u32x4{in ? x.x : 0u, in ? x.y : 0u, in ? x.z : 0u, in ? x.w : 0u};
+      }
+      *(u32x4*)(vw + buf * 1024 + l * 16) = x;
+    };
+    // block j: its lines written two blocks ahead, its operands read one block ahead
+    constexpr int NS = RB / 4;                      // steps per block
+    float va[2][NS][DT], ea[2][NS];
+    auto read_block = [&](int buf, int p, float (&v)[NS][DT], float (&e)[NS]) {
+#pragma unroll
+      for (int i = 0; i < RB / 16; i++) {
+        const f32x4 x = *(const f32x4*)(P + p + 16 * i + 4 * g4);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          e[4 * i + s] = x[s];
+          const uint8_t* y = vw + buf * 1024 + (16 * i + 4 * s + g4) * SB + n16 * kVB;
+#pragma unroll
+          for (int d = 0; d < DT; d++) v[4 * i + s][d] = kF16 ? lt_h2f(((const uint16_t*)y)[d]) : ((const float*)y)[d];
+        }
+      }
+    };
+    put_v(0, vr[0], 0);
+    put_v(1, vr[1], RB);
+    read_block(0, 0, va[0], ea[0]);
+    for (int p = 0; p < nv; p += D * RB) {
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        vr[j] = load_v(p + (j + D) * RB);
+        read_block((j + 1) & 1, p + (j + 1) * RB, va[(j + 1) & 1], ea[(j + 1) & 1]);
+        put_v(j & 1, vr[(j + 2) % D], p + (j + 2) * RB);
+#pragma unroll
+        for (int i = 0; i < NS; i++)
+#pragma unroll
+          for (int d = 0; d < DT; d++)
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[j & 1][i][d], ea[j & 1][i], o[d], 0, 0, 0);
+        if (p + (j + 1) * RB >= nv) break;          // (the rest of the group: zero rows)
+      }
+    }
+  }
+  // the matrix results complete before what reads them in a later block (lt_attn_mm.hip)
+#pragma unroll
+  for (int d = 0; d < DT; d++) asm volatile("s_nop 10" : "+v"(o[d]));
+  __syncthreads();                                  // Z
+  if (w < NP && n16 == 0) {
+    const float z = sm[NW];
+    const float en = kStep && valid ? P[e_slot(len0)] : 0.0f;
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int dim = db + DT * (4 * g4 + r) + d;
+        float x = o[d][r];
+        if (kStep) x = fmaf(en, sv[dim], x);
+        so[dim] = valid ? x / z : 0.0f;
+      }
+  }
+  __syncthreads();
+  const size_t hrow = (size_t)b * A.nh + h;
+  if (A.out && tid < HD) A.out[hrow * HD + tid] = so[tid];
+  if (A.oq && tid < HD) {
+    const size_t blk = q8_out_block(A.obm, A.nh, HD, hrow * (HD / 32) + (tid >> 5));
+    quant_block_hw(so[tid], tid & 31, A.oq + blk * 32, A.od + blk);
+  }
+}
+
+// LDS of 8 waves: vectors, V blocks, K lines, the exps (read up to a block past the last group).
+size_t head_lds(int hd, int maxt) {
+  return (size_t)(4 * hd + 12 + 8 * 512 + 8 * 64 * 36 + ((maxt + 255) & ~255) + 32) * sizeof(float);
+}
+
+}  // namespace
+
+// One workgroup per CU is what the kernel is for: past that its workgroups (76 KB of LDS and up
+// to 256 registers a wave) run one after the other, and the kernels that share a KV group's rows
+// among its heads win.  Per launch, before (k_attn_w1 / k_attn_dec) / here, 14 heads of 64 over 2
+// KV heads: step at 100 / 300 / 600 / 905 rows, fp32 7.7 13.5 21.9 31.0 / 7.6 9.7 12.9 16.2 us, fp16
+// 6.6 10.9 17.7 24.2 / 6.7 8.4 10.6 13.2; batched, up to 500 rows of fp16, 2 / 8 / 16 / 64 sequences
+// 13.9 17.7 17.6 18.0 / 8.5 9.4 9.5 27.9.  32 heads of 128 over 8, step at 905 rows: 71.5 / 20.6.
+bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int hd, int maxt) {
+  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  return (hd == 64 || hd == 128) && (size_t)batch * nh <= (size_t)cus && head_lds(hd, maxt) <= 160 * 1024;
+}
+
+int lt_attn_head(lt_ctx* ctx, LtAttnHead A, int hd, bool f16, bool step) {
+  const size_t shm = head_lds(hd, A.maxt);
+  const dim3 grid((unsigned)((A.batch * A.nkv + 7) / 8 * 8) * (unsigned)(A.nh / A.nkv));
+#define LT_HEAD_CASE(F, H, S)                                                        \
+  if (f16 == F && hd == H && step == S) k_attn_head<F, H, 8, S><<<grid, 512, shm, ctx->stream>>>(A);
+  LT_HEAD_CASE(true, 64, true) LT_HEAD_CASE(false, 64, true) LT_HEAD_CASE(true, 128, true)
+  LT_HEAD_CASE(false, 128, true) LT_HEAD_CASE(true, 64, false) LT_HEAD_CASE(false, 64, false)
+  LT_HEAD_CASE(true, 128, false) LT_HEAD_CASE(false, 128, false)
+#undef LT_HEAD_CASE
+  return lt_check_launch("k_attn_head");
+}

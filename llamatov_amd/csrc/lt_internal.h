@@ -86,6 +86,27 @@ struct LtAttnMm {
 bool lt_attn_mm_covers(int hd, int T, int maxt, int nsplit);
 int lt_attn_mm_prefill(lt_ctx* ctx, LtAttnMm A, int hd, bool f16);
 
+// Unsplit decode attention, one workgroup per (head, sequence) (lt_attn_head.hip): the decode
+// step (qkv, freqs; one sequence) or batched decode (q rows q_stride floats apart).
+struct LtAttnHead {
+  const float* qkv;
+  const float* freqs;
+  const float* q;
+  int q_stride;
+  void* kc;
+  void* vc;
+  const int* len;
+  float* out;
+  int8_t* oq;
+  uint16_t* od;
+  int obm;
+  int batch, nh, nkv;
+  float scale;
+  int maxt;
+};
+bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int hd, int maxt);
+int lt_attn_head(lt_ctx* ctx, LtAttnHead A, int hd, bool f16, bool step);
+
 // Device helpers shared by the kernel translation units.
 __device__ __forceinline__ float lt_h2f(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));

@@ -362,4 +362,14 @@ __device__ __forceinline__ void build_act_records(const int8_t* sxq, const uint1
   }
 }
 
+// Where block g of the quantized output goes (g counts the blocks of the [rows][nh*hd] output
+// row by row): row-major, or with obm > 0 block-major over obm rows -- quants [nh*hd/32][obm]
+// [32], scales [nh*hd/32][obm], the tiled GEMM's activation layout.
+__device__ __forceinline__ size_t q8_out_block(int obm, int nh, int hd, size_t g) {
+  if (obm <= 0) return g;
+  const size_t nbr = (size_t)(nh * hd / 32);
+  const size_t row = g / nbr;
+  return (g - row * nbr) * (size_t)obm + row;
+}
+
 }  // namespace lt
