@@ -1086,15 +1086,30 @@ int check_gemm(const char* fn, const void* W, const int8_t* Xq, const uint16_t* 
   return LT_OK;
 }
 
-// LT_GEMM_LS=0 keeps every launch on k_q8_gemm (for comparisons), 1 sends every tiled launch
-// to the leaf-split kernel.  By default a tiled launch takes it when it holds at most kLsMaxT
-// tokens, or when k_q8_gemm's grid (kGemmTokens-token tiles) would hold fewer than kLsFill
-// workgroups per CU: there the leaf-split kernel's 32-token tiles, four waves each, fill the
-// chip.  Measured per launch, k_q8_gemm / leaf-split (us): 896 x 4864 at T = 512 40.5 / 15.4,
-// 1152 x 896 at 512 19.7 / 10.6, 9728 x 896 at 128 22.1 / 18.4 but at 256 28.3 / 31.7,
-// 4096 x 4096 at 256 30.6 / 27.7 but at 512 40.7 / 46.6, 151936 x 896 at 128 169 / 206.
-constexpr int kLsMaxT = 64;
-constexpr int kLsFill = 2;
+// Which tiled launches take the leaf-split kernel (LT_GEMM_LS=0 / 1 forces k_q8_gemm / the
+// leaf-split kernel, read at every launch).  k_q8_gemm's tiles are 128 tokens, one 32 x 32 tile a
+// wave, with the fewest instructions where K % 2048 == 0 lets its leaves go in static groups; the
+// leaf-split kernel's are 32 tokens, 4 to 16 waves a tile, its schedule fixed at compile time up to
+// 5 blocks a leaf.  Measured per launch over rotated weight copies, k_q8_gemm / leaf-split (us):
+//  - one block per leaf (K <= 1024), any size: k_q8_gemm walks run-time leaves of one block there:
+//    9728 x 896 at T = 256 / 509 / 2048 24.5 / 15.6, 40.9 / 25.6, 134 / 84.8; 151936 x 896 at 128
+//    and 256 137 / 85, 281 / 198; 1152 x 896 at 2048 27.1 / 15.9;
+//  - two (K <= 2048): unless the grouped walk applies and has 3 waves per SIMD: 11008 x 2048 at 256
+//    and 512 27.4 / 28.9, 46.8 / 51.1; 2048 x 2048 at 512 18.7 / 14.7;
+//  - three to five (K <= 5120): up to 128 tokens and while k_q8_gemm's grid holds less than 2
+//    workgroups per CU: 28672 x 4096 at 32 / 64 / 128 / 256 61 / 33, 63 / 44, 69 / 71, 116 / 127;
+//    6144 x 4096 at 256 / 400 33.9 / 32.4, 41.9 / 47.0; 4096 x 4096 at 256 / 512 29.7 / 23.0, 36.2 /
+//    40.2; 896 x 4864 at 509 and 1024 41.7 / 11.9, 46 / 26.9;
+//  - more: up to 64 tokens or on the same grids: 4096 x 14336 at 64 / 256 / 400 / 512 95 / 24.7, 95 /
+//    71, 107 / 103, 109 / 118.
+bool take_ls(const lt_ctx* ctx, const GemmParams& P) {
+  const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const long wgs = (long)((P.nrt + 7) / 8) * 8 * ((P.T + kGemmTokens - 1) / kGemmTokens);
+  const int bpl = (P.K / 32 + 31) / 32;             // blocks per leaf
+  if (bpl == 1) return true;
+  if (bpl == 2) return !(P.K % 2048 == 0 && (long)P.nrt * ((P.T + 31) / 32) >= 12 * cus);
+  return P.T <= (bpl <= 5 ? 128 : 64) || wgs < 2 * cus;
+}
 int ls_mode() {
   const char* s = getenv("LT_GEMM_LS");
   return s ? atoi(s) : -1;
@@ -1130,23 +1145,21 @@ int launch_gemm(lt_ctx* ctx, GemmParams P) {
   P.nrt = (P.N + 31) / 32;
   if constexpr (kTiled) {
     const int mode = ls_mode();
-    const long wgs = (long)((P.nrt + 7) / 8) * 8 * ((P.T + kGemmTokens - 1) / kGemmTokens);
-    const long fill = (long)kLsFill * (ctx->num_cus > 0 ? ctx->num_cus : 256);
-    if (mode == 1 || (mode < 0 && (P.T <= kLsMaxT || wgs < fill))) {
+    if (mode == 1 || (mode < 0 && take_ls(ctx, P))) {
       P.ntt = (P.T + 31) / 32;
       const long gls = (long)((P.nrt + 7) / 8) * 8 * P.ntt;
-      // 8 waves per tile when the launch holds at most one tile per CU, 16 when in addition
-      // each leaf holds 3 to 5 blocks (K 2049 .. 5120; LT_GEMM_LS_W=4 / 8 / 16 forces one,
-      // read at every launch).  Measured at T = 64, 4 / 8 waves (us): 896 x 4864 13.4 / 8.9,
-      // 896 x 896 7.9 / 5.6, 4096 x 4096 13.1 / 10.3, 4096 x 14336 29.4 / 24.7, but 6144 x
-      // 4096 15.2 / 17.4 and 9728 x 896 10.8 / 14.0 (384 and 608 tiles); 8 / 16 waves on the
-      // compile-time schedule: 896 x 4864 7.95 / 7.58, 4096 x 4096 9.52 / 9.12, 896 x 896
-      // 4.19 / 4.26.
+      // Waves per tile (LT_GEMM_LS_W=4 / 8 / 16 forces one, read at every launch).  At most one
+      // tile per CU: 8, and 16 when each leaf holds 3 to 5 blocks (T = 64, 8 / 16 waves: 896 x
+      // 4864 7.95 / 7.58 us, 4096 x 4096 9.52 / 9.12, 896 x 896 4.19 / 4.26).  More tiles: 4,
+      // but 8 where that is what fits the compile-time schedule, 3 to 5 blocks (4 / 8 waves:
+      // 896 x 4864 at T = 509 17.8 / 12.9, 6144 x 4096 at 64 and 256 14.4 / 10.4, 33.9 / 25.0, 28672
+      // x 4096 at 64 38.3 / 30.8; one block: 9728 x 896 at 509 24.8 / 30.2).
       const char* wenv = getenv("LT_GEMM_LS_W");
       const int wforce = wenv ? atoi(wenv) : 0;
       const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
       const int bpl = (P.K / 32 + 31) / 32;
-      const int w = wforce ? wforce : gls > cus ? 4 : (bpl >= 3 && bpl <= 5) ? 16 : 8;
+      const bool mid = bpl >= 3 && bpl <= 5;
+      const int w = wforce ? wforce : gls > cus ? (mid ? 8 : 4) : mid ? 16 : 8;
       if (w == 16) launch_ls<EPI, 16, false>(ctx, P, (unsigned)gls);
       else if (w == 8) launch_ls<EPI, 8, false>(ctx, P, (unsigned)gls);
       else launch_ls<EPI, 4, false>(ctx, P, (unsigned)gls);
@@ -1156,17 +1169,24 @@ int launch_gemm(lt_ctx* ctx, GemmParams P) {
   P.ntt = (P.T + kGemmTokens - 1) / kGemmTokens;
   const long grid = (long)((P.nrt + 7) / 8) * 8 * P.ntt;
   if constexpr (kTiled) {
-    // K a multiple of 2048 (an even number of blocks per leaf, bpl): grouped leaves -- with a
-    // 2-slot ring when the launch holds 3 or more waves per SIMD (the other waves hide the
-    // latency), else (bpl % 4 == 0) with a 4-slot ring and pipelined MFMAs in 256 registers.
+    // K a multiple of 2048 (an even number of blocks per leaf, bpl): grouped leaves.  The 2-slot
+    // ring keeps 3 waves per SIMD (the other waves hide the latency), the 4-slot ring with
+    // pipelined MFMAs 2 (bpl % 4 == 0): a resident round of the latter takes about 0.8 of the
+    // former's time, so the rounds decide (2-slot / 4-slot, us: 4096 x 4096 at 512 and 1024 tokens
+    // 41.2 / 36.2, 80.3 / 68.2; 6144 x 4096 at 400 and 512 41.9 / 54.0, 44.2 / 55.8; 28672 x 4096 at
+    // 128 / 512 81 / 69, 203 / 215).  Other bpl: the 2-slot ring where it fills the chip, but not
+    // past 8 blocks a leaf (4096 x 14336 at 512 and 1024, dynamic / 2-slot 109 / 119, 220 / 239).
     // LT_GEMM_GROUPED=0 / 1 / 2 forces the dynamic walk / the 2-slot / the 4-slot walk where
     // K allows it (read at every launch).
     if (P.K % 2048 == 0) {
       const int bpl = P.K / 1024;
       const long waves = (long)P.nrt * ((P.T + 31) / 32);
-      const bool big = waves >= 12L * (ctx->num_cus > 0 ? ctx->num_cus : 256);
+      const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+      const long r2 = (waves + 12 * cus - 1) / (12 * cus), r4 = (waves + 8 * cus - 1) / (8 * cus);
       const char* force = getenv("LT_GEMM_GROUPED");
-      const int walk = force ? atoi(force) : big ? 1 : bpl % 4 == 0 ? 2 : 0;
+      const int walk = force                ? atoi(force)
+                       : bpl % 4 == 0       ? (4 * r4 < 5 * r2 ? 2 : 1)
+                       : bpl <= 8 && waves >= 12 * cus ? 1 : 0;
       if (walk == 1) {
         k_q8_gemm<EPI, true, 1><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
         return lt_check_launch("k_q8_gemm");
