@@ -1656,7 +1656,7 @@ int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, 
   if (mm) return launch_mm();
   if ((mode == AM_STEP || mode == AM_DECODE) && A.nsplit == 1 && use_head() &&
       (w1 || ((size_t)hpw * A.hd + 2 * A.hd + (size_t)hpw * per_max + kVChunkFloats) * sizeof(float) <= 64 * 1024) &&
-      lt_attn_head_covers(ctx, rows, A.nh, A.hd, A.maxt)) {
+      lt_attn_head_covers(ctx, rows, A.nh, A.nkv, A.hd, A.maxt, mode == AM_STEP)) {
     LtAttnHead H = {};
     H.qkv = A.qkv; H.freqs = A.freqs; H.q = A.q; H.q_stride = A.q_stride; H.kc = A.kc; H.vc = A.vc; H.len = A.len;
     H.out = A.out; H.oq = A.oq; H.od = A.od; H.obm = A.obm; H.batch = rows; H.nh = A.nh; H.nkv = A.nkv;

@@ -15,6 +15,8 @@
 //            operands are read from LDS a block ahead.
 // K rows are requested before the length is known; V rows past it are replaced by zeros.
 //
+// k_attn_group below does the same with a workgroup per KV group for grids of more heads than CUs.
+//
 // The heads of a KV group run on one XCD (workgroups are dealt to the 8 XCDs round-robin), so a
 // group's rows are fetched into one L2 once.
 #include "lt_q8_device.h"
@@ -22,8 +24,6 @@
 namespace {
 
 using namespace lt;
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Position t's slot in the exps: a lane of group k reads its four steps' exps (t = 4 i + k, i =
 // 0..3) of a 16-position tile as one 16-byte word.
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
         for (int i = 0; i < NS; i++)
 #pragma unroll
           for (int d = 0; d < DT; d++)
-            o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[j & 1][i][d], ea[j & 1][i], o[d], 0, 0, 0);
+            o[d] = mma(va[j & 1][i][d], ea[j & 1][i], o[d]);
         if (p + (j + 1) * RB >= nv) break;          // (the rest of the group: zero rows)
       }
     }
@@ -291,25 +291,258 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
   }
 }
 
+// Batched decode past one head per CU: a workgroup of 8 waves takes all heads of one KV group of
+// one sequence, so its cache rows are read and converted once.  The heads are the columns of the
+// matrix instructions (16, of which nh / nkv are used):
+//   scores   tiles of 16 positions as in k_attn_mm, a wave every eighth tile, two tiles in flight;
+//            a lane's four scores lie side by side by e_slot;
+//   softmax  a wave per head: exps four at a time, Z by the 64-lane fold and tree;
+//   O        as above with each head's exps in its own column, a wave per 16 dims.
+// Bound by the serial chain over the positions and by one wave's exps; at most one workgroup runs
+// per CU, so registers are not short.
+template <bool kF16, int HD>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_attn_group(LtAttnHead A, int cap) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  constexpr int NW = 8;
+  constexpr int kEb = kF16 ? 2 : 4;
+  constexpr int NU = HD * kEb / 64;                 // 16-byte units per lane and K tile
+  constexpr int NP = HD / 16;                       // waves that fold O, 16 dims each
+  constexpr int SB = 16 * kEb;
+  constexpr int RB = 1024 / SB;
+  constexpr int D = 256 / RB;
+  static_assert(NP <= NW, "k_attn_group: head size");
+  const int rep = A.nh / A.nkv, ps = cap + 4;
+  float* sm = lds;                                  // [NW][16] maxima, [16] Z
+  uint8_t* vbuf = (uint8_t*)(sm + NW * 16 + 16);    // [NP][2][1024]
+  float* P = (float*)(vbuf + NP * 2048);            // [rep][ps] exps by e_slot; then the outputs
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+  const int n16 = l & 15, g4 = l >> 4;
+  const int b = (int)blockIdx.x / A.nkv, g = (int)blockIdx.x - b * A.nkv;
+  const int len0 = A.len[b];
+  const uint32_t pitch = (uint32_t)A.nkv * HD * kEb;
+  const size_t seq = (size_t)b * A.maxt * pitch;
+  const uint32_t gb = (uint32_t)g * HD * kEb;
+  const int seq_end = (int)((uint32_t)A.maxt * pitch);
+  const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)A.kc + seq, 0, seq_end, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc((uint8_t*)A.vc + seq, 0, seq_end, 0x00020000);
+
+  // K tile at position p: unit 4 j + g4 of the row that makes matrix row n16 position 4 (n16 & 3) +
+  // n16 / 4, so that a lane's four scores lie side by side by e_slot
+  const uint32_t kb0 = gb + (uint32_t)((n16 & 3) * 4 + (n16 >> 2)) * pitch + (uint32_t)g4 * 16u;
+  auto load_unit = [&](int p, int j) {
+    return __builtin_amdgcn_raw_buffer_load_b128(krsrc, (int)(kb0 + (uint32_t)p * pitch + 64u * j), 0, 0);
+  };
+  u32x4 kb[2][NU];
+#pragma unroll
+  for (int j = 0; j < NU; j++) kb[0][j] = load_unit(w * 16, j);      // (before the length)
+  float qr[HD / 4];
+  {
+    const float* qs = A.q + (size_t)b * A.q_stride + (size_t)(g * rep + (n16 < rep ? n16 : 0)) * HD;
+#pragma unroll
+    for (int j = 0; j < HD / 16; j++) {
+      const u32x4_a4 x = *(const u32x4_a4*)(qs + 16 * j + 4 * g4);
+      uint32_t r[4] = {x.x, x.y, x.z, x.w};
+      transpose4(r);
+#pragma unroll
+      for (int e = 0; e < 4; e++) qr[4 * j + e] = __uint_as_float(r[e]);
+    }
+  }
+  const int n = len0 < 0 ? 0 : (len0 > A.maxt ? A.maxt : len0);
+  if ((w + NW) * 16 < n) {
+#pragma unroll
+    for (int j = 0; j < NU; j++) kb[1][j] = load_unit((w + NW) * 16, j);
+  }
+
+  float mx = -1e30f;
+  for (int p = w * 16; p < n; p += 32 * NW) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int pi = p + 16 * NW * i;
+      if (pi < n) {
+        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < NU; j++) {
+          const u32x4 k = kb[i][j];
+          if (kF16) {
+            uint32_t r[4] = {__builtin_amdgcn_perm(k.z, k.x, 0x05040100u), __builtin_amdgcn_perm(k.z, k.x, 0x07060302u),
+                             __builtin_amdgcn_perm(k.w, k.y, 0x05040100u), __builtin_amdgcn_perm(k.w, k.y, 0x07060302u)};
+            if (pi + 32 * NW < n) kb[i][j] = load_unit(pi + 32 * NW, j);
+            transpose4(r);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              s = mma(lt_h2f((uint16_t)(r[e] & 0xFFFFu)), qr[8 * j + 2 * e], s);
+              s = mma(lt_h2f((uint16_t)(r[e] >> 16)), qr[8 * j + 2 * e + 1], s);
+            }
+          } else {
+            uint32_t r[4] = {k.x, k.y, k.z, k.w};
+            if (pi + 32 * NW < n) kb[i][j] = load_unit(pi + 32 * NW, j);
+            transpose4(r);
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = mma(__uint_as_float(r[e]), qr[4 * j + e], s);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          s[r] = s[r] * A.scale;
+          if (pi + 4 * r + g4 < n) mx = fmaxf(mx, s[r]);
+        }
+        if (n16 < rep) *(f32x4*)(P + n16 * ps + pi + 4 * g4) = s;
+      }
+    }
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  if (l < 16) sm[w * 16 + l] = mx;
+  // V block at row p: this wave's 16 dims
+  const int vrow = l / (SB / 16);
+  const uint32_t vb = gb + (uint32_t)(w < NP ? w : 0) * SB + (uint32_t)(l % (SB / 16)) * 16u;
+  auto load_v = [&](int p) {
+    return __builtin_amdgcn_raw_buffer_load_b128(vrsrc, (int)((uint32_t)(p + vrow) * pitch + vb), 0, 0);
+  };
+  u32x4 vr[D];
+  if (w < NP) {
+#pragma unroll
+    for (int j = 0; j < D; j++)
+      if (j < 2 || j * RB < n) vr[j] = load_v(j * RB);
+  }
+  __syncthreads();
+  // lane l takes positions l, l + 64, ..., four at a time; zeros up to whole groups of the O loop
+  const int n_up = (n + 255) & ~255;
+  for (int h = w; h < rep; h += NW) {
+    float m = -1e30f;
+#pragma unroll
+    for (int i = 0; i < NW; i++) m = fmaxf(m, sm[i * 16 + h]);
+    float z = 0.0f;
+    for (int t0 = 0; t0 < n_up; t0 += 256) {
+      float* pe = P + h * ps + t0 + e_slot(l);
+      auto part = [&](auto N) {                     // exps of the first N of the four
+        float e[4] = {0.0f, 0.0f, 0.0f, 0.0f}, x[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) x[u] = pe[64 * u] - m;
+        lt_expf_n(x);
+#pragma unroll
+        for (int u = 0; u < N; u++) e[u] = t0 + 64 * u + l < n ? x[u] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          pe[64 * u] = e[u];
+          if (u < N) z = z + e[u];
+        }
+      };
+      if (n - t0 > 64) part(std::integral_constant<int, 4>{});
+      else part(std::integral_constant<int, 1>{});
+    }
+    z = wave_tree_dpp(z);
+    if (l == 0) sm[NW * 16 + h] = z;
+  }
+  __syncthreads();
+  f32x4 o[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
+  if (w < NP) {
+    uint8_t* const vw = vbuf + w * 2048;
+    const float* pb = P + (n16 < rep ? n16 : 0) * ps + 4 * g4;
+    auto put_v = [&](int buf, u32x4 x, int p) {
+      if (p + RB > n) {                             // rows past the length may hold anything
+        const bool in = p + vrow < n;
+        x = u32x4{in ? x.x : 0u, in ? x.y : 0u, in ? x.z : 0u, in ? x.w : 0u};
+      }
+      *(u32x4*)(vw + buf * 1024 + l * 16) = x;
+    };
+    constexpr int NS = RB / 4;
+    float va[2][NS], ea[2][NS];
+    auto read_block = [&](int buf, int p, float (&v)[NS], float (&e)[NS]) {
+#pragma unroll
+      for (int i = 0; i < RB / 16; i++) {
+        const f32x4 x = *(const f32x4*)(pb + p + 16 * i);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          e[4 * i + s] = x[s];
+          const uint8_t* y = vw + buf * 1024 + (16 * i + 4 * s + g4) * SB + n16 * kEb;
+          v[4 * i + s] = kF16 ? lt_h2f(*(const uint16_t*)y) : *(const float*)y;
+        }
+      }
+    };
+    put_v(0, vr[0], 0);
+    put_v(1, vr[1], RB);
+    read_block(0, 0, va[0], ea[0]);
+    for (int p = 0; p < n; p += D * RB) {
+#pragma unroll
+      for (int j = 0; j < D; j++) {
+        vr[j] = load_v(p + (j + D) * RB);
+        read_block((j + 1) & 1, p + (j + 1) * RB, va[(j + 1) & 1], ea[(j + 1) & 1]);
+        put_v(j & 1, vr[(j + 2) % D], p + (j + 2) * RB);
+#pragma unroll
+        for (int i = 0; i < NS; i++) o[0] = mma(va[j & 1][i], ea[j & 1][i], o[0]);
+        if (p + (j + 1) * RB >= n) break;           // (the rest of the group: zero rows)
+      }
+    }
+  }
+  // the matrix results complete before what reads them in a later block (lt_attn_mm.hip)
+  asm volatile("s_nop 10" : "+v"(o[0]));
+  __syncthreads();                                  // the exps are free
+  float* so = P;                                    // [rep][HD]
+  if (w < NP && n16 < rep) {
+    const float z = sm[NW * 16 + n16];
+#pragma unroll
+    for (int r = 0; r < 4; r++) so[n16 * HD + w * 16 + 4 * g4 + r] = o[0][r] / z;
+  }
+  __syncthreads();
+  const size_t hrow = (size_t)b * A.nh + (size_t)g * rep;
+  for (int i = tid; i < rep * HD; i += 512) {       // (whole half-waves: HD is a multiple of 32)
+    if (A.out) A.out[hrow * HD + i] = so[i];
+    if (A.oq) {
+      const size_t blk = q8_out_block(A.obm, A.nh, HD, hrow * (HD / 32) + (i >> 5));
+      quant_block_hw(so[i], i & 31, A.oq + blk * 32, A.od + blk);
+    }
+  }
+}
+
 // LDS of 8 waves: vectors, V blocks, K lines, the exps (read up to a block past the last group).
 size_t head_lds(int hd, int maxt) {
   return (size_t)(4 * hd + 12 + 8 * 512 + 8 * 64 * 36 + ((maxt + 255) & ~255) + 32) * sizeof(float);
 }
 
+int group_cap(int maxt) { return (maxt + 255) & ~255; }
+size_t group_lds(int hd, int rep, int maxt) {
+  const size_t exps = (size_t)rep * (group_cap(maxt) + 4) + 64, outs = (size_t)rep * hd;
+  return (size_t)(8 * 16 + 16 + hd / 16 * 512 + (exps > outs ? exps : outs)) * sizeof(float);
+}
+
 }  // namespace
 
-// One workgroup per CU is what the kernel is for: past that its workgroups (76 KB of LDS and up
-// to 256 registers a wave) run one after the other, and the kernels that share a KV group's rows
-// among its heads win.  Per launch, before (k_attn_w1 / k_attn_dec) / here, 14 heads of 64 over 2
-// KV heads: step at 100 / 300 / 600 / 905 rows, fp32 7.7 13.5 21.9 31.0 / 7.6 9.7 12.9 16.2 us, fp16
-// 6.6 10.9 17.7 24.2 / 6.7 8.4 10.6 13.2; batched, up to 500 rows of fp16, 2 / 8 / 16 / 64 sequences
-// 13.9 17.7 17.6 18.0 / 8.5 9.4 9.5 27.9.  32 heads of 128 over 8, step at 905 rows: 71.5 / 20.6.
-bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int hd, int maxt) {
-  const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  return (hd == 64 || hd == 128) && (size_t)batch * nh <= (size_t)cus && head_lds(hd, maxt) <= 160 * 1024;
+// One workgroup per CU is what both kernels are for: k_attn_head (76 KB of LDS, up to 256
+// registers a wave) takes the grids of at most one head per CU, k_attn_group those of more heads
+// but at most one KV group per CU, up to its 16 matrix rows.  Past that the workgroups run one
+// after the other and the smaller ones of lt_attn.hip are as fast or faster: 512 groups of 2 heads
+// of 64, up to 500 rows of fp16, 18.4 us there, 19.6 here; 512 of 4 heads of 128 25.2 / 32.4.
+//
+// Per launch, before (k_attn_w1 / k_attn_dec) / here, in us.  k_attn_head, 14 heads of 64 over 2 KV
+// heads: step at 100 / 300 / 600 / 905 rows, fp32 7.7 13.5 21.9 31.0 / 7.6 9.7 12.9 16.2, fp16 6.6
+// 10.9 17.7 24.2 / 6.7 8.4 10.6 13.2; batched, up to 500 rows of fp16, 2 / 8 / 16 sequences 13.9
+// 17.7 17.6 / 8.5 9.4 9.5.  32 heads of 128 over 8, step at 905 rows: 71.5 / 20.6.
+// k_attn_group, fp16, 64 sequences of up to 40 / 100 / 200 / 500 rows of the 14 heads: 5.5 7.2 10.7
+// 18.0 / 6.1 7.3 9.1 13.4 (the length is not known at the launch; 27.9 with k_attn_head), fp32 at
+// 500 19.9 / 15.3; 32 heads of 128 over 8, 16 sequences: fp16 at 500 20.4 / 18.5, fp32 at 700 59.7 /
+// 27.3.
+static bool fits_cus(const lt_ctx* ctx, int batch, int heads) {
+  return (size_t)batch * heads <= (size_t)(ctx->num_cus > 0 ? ctx->num_cus : 256);
+}
+
+bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int nkv, int hd, int maxt, bool step) {
+  if (hd != 64 && hd != 128) return false;
+  if (fits_cus(ctx, batch, nh)) return head_lds(hd, maxt) <= 160 * 1024;
+  return !step && fits_cus(ctx, batch, nkv) && nh / nkv <= 16 && (size_t)maxt * nkv * hd * 4 < ((size_t)1 << 31) &&
+         group_lds(hd, nh / nkv, maxt) <= 160 * 1024;
 }
 
 int lt_attn_head(lt_ctx* ctx, LtAttnHead A, int hd, bool f16, bool step) {
+  if (!fits_cus(ctx, A.batch, A.nh)) {
+    const size_t shm = group_lds(hd, A.nh / A.nkv, A.maxt);
+    const unsigned grid = (unsigned)A.batch * (unsigned)A.nkv;
+#define LT_GROUP_CASE(F, H) \
+  if (f16 == F && hd == H) k_attn_group<F, H><<<grid, 512, shm, ctx->stream>>>(A, group_cap(A.maxt));
+    LT_GROUP_CASE(true, 64) LT_GROUP_CASE(false, 64) LT_GROUP_CASE(true, 128) LT_GROUP_CASE(false, 128)
+#undef LT_GROUP_CASE
+    return lt_check_launch("k_attn_group");
+  }
   const size_t shm = head_lds(hd, A.maxt);
   const dim3 grid((unsigned)((A.batch * A.nkv + 7) / 8 * 8) * (unsigned)(A.nh / A.nkv));
 #define LT_HEAD_CASE(F, H, S)                                                        \

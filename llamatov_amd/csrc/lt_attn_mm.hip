@@ -39,23 +39,7 @@ namespace {
 
 using namespace lt;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr uint32_t kNoRow = 0x80000000u;   // out-of-range buffer offset: reads zeros
-
-__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// 4 x 4 transpose of four registers over the four 16-lane groups: group g's register r becomes
-// group r's register g.
-__device__ __forceinline__ void transpose4(uint32_t (&r)[4]) {
-  const u32x2 a = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
-  const u32x2 b = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
-  const u32x2 c = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false);
-  const u32x2 d = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
-  r[0] = c.x; r[1] = c.y; r[2] = d.x; r[3] = d.y;
-}
 
 // Whether one of a dword's values (two fp16 or one fp32) is not finite.
 __device__ __forceinline__ int not_finite_bits(uint32_t w, bool f16) {

@@ -104,7 +104,7 @@ struct LtAttnHead {
   float scale;
   int maxt;
 };
-bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int hd, int maxt);
+bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int nkv, int hd, int maxt, bool step);
 int lt_attn_head(lt_ctx* ctx, LtAttnHead A, int hd, bool f16, bool step);
 
 // Device helpers shared by the kernel translation units.

@@ -135,7 +135,7 @@ __device__ __forceinline__ float wave_max(float a) {
 // lt_expf_sel of N values at once, written stage by stage so that the N binary64 chains
 // interleave, and held straight-line: the compiler otherwise turns lt_expf_sel's selects into
 // branches around its polynomial and runs one value after the other (attention's softmax, four
-// values a lane: 1470 -> 700 cycles).  Equal to lt_expf_sel for every input (a nan is clamped
+// values a lane: 1470 -> 960 cycles).  Equal to lt_expf_sel for every input (a nan is clamped
 // to -120 here and put back by the last select).
 template <int N>
 __device__ __forceinline__ void lt_expf_n(float (&x)[N]) {
@@ -370,6 +370,26 @@ __device__ __forceinline__ size_t q8_out_block(int obm, int nh, int hd, size_t g
   const size_t nbr = (size_t)(nh * hd / 32);
   const size_t row = g / nbr;
   return (g - row * nbr) * (size_t)obm + row;
+}
+
+// ---- fp32 matrix instructions ----------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// D[i][j] = C[i][j] + sum over k = 0..3 of A[i][k] B[k][j], the four products added one after the
+// other in ascending k, each with one rounding (lt_attn_mm.hip).  Lane (n, g) = (lane & 15, lane >>
+// 4) gives A[n][g] and B[g][n] and holds D[4 g + r][n] in register r.
+__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// 4 x 4 transpose of four registers over the four 16-lane groups: group g's register r becomes
+// group r's register g.
+__device__ __forceinline__ void transpose4(uint32_t (&r)[4]) {
+  const u32x2 a = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+  const u32x2 b = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+  const u32x2 c = __builtin_amdgcn_permlane16_swap(a.x, b.x, false, false);
+  const u32x2 d = __builtin_amdgcn_permlane16_swap(a.y, b.y, false, false);
+  r[0] = c.x; r[1] = c.y; r[2] = d.x; r[3] = d.y;
 }
 
 }  // namespace lt

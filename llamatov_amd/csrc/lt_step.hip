@@ -38,8 +38,6 @@ namespace {
 
 using namespace lt;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int kT = 256;                 // threads per workgroup
 constexpr int kHd = 64;                 // head size
 constexpr int kMaxE = 1024;             // n_embd and n_head*hd: one 32-block item per row

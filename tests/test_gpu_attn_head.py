@@ -1,8 +1,10 @@
 """Unsplit decode attention with a workgroup per head (lt_attn_head.hip) at the lengths where it
 can go wrong, against the oracle bit for bit: the 64-position score rounds and their spread over 8
 waves (512 positions, 1024), the 16- and 32-row V blocks and the 256 rows in flight, both cache
-types and head sizes, the step's new row at each of those places, nan past the length, and a batch
-of as many (sequence, head) pairs as there are CUs and one more sequence."""
+types and head sizes, the step's new row at each of those places, nan past the length; batches of as
+many (sequence, head) pairs as there are CUs and one more sequence; and past that a workgroup per KV
+group (2 to 16 heads, tiles of 16 positions, 128 and 256 of them in flight) and the first groups
+that it leaves to the general kernel (17 heads, more groups than CUs)."""
 import ctypes
 
 import numpy as np
@@ -54,7 +56,8 @@ def test_step_lengths(gpu, oracle, kv_dtype, nh, nkv, hd):
 
 
 @pytest.mark.parametrize("kv_dtype", [LT_KV_F32, LT_KV_F16])
-@pytest.mark.parametrize("nh,nkv,hd,B", [(14, 2, 64, 16), (4, 1, 128, 16), (64, 8, 64, 4), (64, 8, 64, 5)])
+@pytest.mark.parametrize("nh,nkv,hd,B", [(14, 2, 64, 16), (4, 1, 128, 16), (64, 8, 64, 4), (64, 8, 64, 5),
+                                          (14, 2, 64, 20), (32, 2, 128, 10), (8, 4, 64, 40), (80, 80, 64, 4), (51, 3, 64, 6)])
 def test_batched_lengths(gpu, oracle, kv_dtype, nh, nkv, hd, B):
     f16, maxt = kv_dtype == LT_KV_F16, 1300
     rng = np.random.default_rng(B * hd)
