@@ -516,10 +516,14 @@ size_t mm_lds(int cap, int nsplit) {
 
 // Splits cost a merge of the chains per split and tile whatever the length, so short prompts
 // stay on the per-row kernel (16 splits, 32 heads of 128, maxt 1024, per-row / here: T = 100
-// 19.0 / 22.3 us, 200 28.7 / 42.3, 512 106 / 95, and at maxt 512 87 / 71).
+// 19.0 / 22.3 us, 200 28.7 / 42.3, 512 106 / 95, and at maxt 512 87 / 71).  So do caches of at most
+// 32 rows of 128: one score tile or two leave most waves idle (32 heads, T = 16 and 32, fp16 7.3 /
+// 8.0 and 7.4 / 8.1, fp32 6.7 / 8.2 and 7.2 / 8.7; at 48 rows 9.5 / 8.7 and 9.6 / 9.1; heads of 64
+// are even from T = 8 on).
 bool lt_attn_mm_covers(int hd, int T, int maxt, int nsplit) {
   if (hd != 64 && hd != 128) return false;
-  return nsplit == 1 || (nsplit % 16 == 0 && T >= 384 && mm_lds((maxt + 63) & ~63, nsplit) <= (size_t)kLds);
+  if (nsplit == 1) return hd == 64 || maxt > 32;
+  return (nsplit % 16 == 0 && T >= 384 && mm_lds((maxt + 63) & ~63, nsplit) <= (size_t)kLds);
 }
 
 int lt_attn_mm_prefill(lt_ctx* ctx, LtAttnMm A, int hd, bool f16) {
