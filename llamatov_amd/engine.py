@@ -1209,11 +1209,14 @@ class PrefillBuffers:
         self.v = DevTensor.empty((T, F), np.float32, D)
         self.xq = DevTensor.empty((T * kmax,), np.int8, D)
         self.xd = DevTensor.empty((T * kmax // 32,), np.uint16, D)
+        self.vq = DevTensor.empty((T * F,), np.int8, D)
+        self.vd = DevTensor.empty((T * F // 32,), np.uint16, D)
         aw = _lib.raw("lt_attn_workspace_size")(T, cfg.n_head, cfg.head_dim, plan.profile.attn_nsplit)
         self.ws = DevTensor.empty((aw,), np.uint8, D) if aw else None
 
     def free(self) -> None:
-        for t in (self.toks, self.x, self.xres, self.qkv, self.att, self.v, self.xq, self.xd, self.ws):
+        for t in (self.toks, self.x, self.xres, self.qkv, self.att, self.v, self.xq, self.xd, self.vq, self.vd,
+                  self.ws):
             if t is not None:
                 t.free()
 
@@ -1272,6 +1275,15 @@ def forward_prefill(plan: DecodePlan, tokens, embeddings: np.ndarray | None = No
          cfg.vocab, E, plan.tok.vp, None, None, 0, plan.am_ws.vp, plan.am_ws.nbytes)
 
 
+# up to this width and this many tokens a prefill's gate|up launch also quantizes its SiLU output
+# (lt_q8_gemm_silu_quant_t), which spares a launch and the fp32 round trip; wider, the kernel that
+# walks K in one go per row tile loses more than that.  Cold weights, two launches / one (us): 9728 x
+# 896 at T = 16 8.2 / 6.4, 64 9.9 / 9.2, 256 19.0 / 17.2, 509 30.6 / 30.3; 28672 x 4096 at T = 8 30.9
+# / 31.0, 64 46.8 / 58.1, 512 210 / 347
+SILU_QUANT_MAX_EMBD = 1024
+SILU_QUANT_MAX_T = 512
+
+
 def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, caches: list, maxt: int,
                     scale: float) -> None:
     """The layers of a batched prefill of the T rows in B.x, one sequence: caches[il] =
@@ -1291,9 +1303,14 @@ def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, cac
         call("lt_quant_q8_bm", h, B.att.vp, B.xq.vp, B.xd.vp, T, QD)
         call("lt_q8_gemm_t", h, L["wo_t"].t.vp, B.xq.vp, B.xd.vp, None, B.x.vp, B.xres.vp, T, E, QD)
         call("lt_rmsnorm_quant_bm", h, B.xres.vp, L["ffn_norm"].vp, B.xq.vp, B.xd.vp, T, E, eps)
-        call("lt_q8_gemm_silu_t", h, L["wgu_il_t"].t.vp, B.xq.vp, B.xd.vp, B.v.vp, T, F, E)
-        call("lt_quant_q8_bm", h, B.v.vp, B.xq.vp, B.xd.vp, T, F)
-        call("lt_q8_gemm_t", h, L["wdown_t"].t.vp, B.xq.vp, B.xd.vp, None, B.xres.vp, B.x.vp, T, E, F)
+        if E <= SILU_QUANT_MAX_EMBD and T <= SILU_QUANT_MAX_T and F % 32 == 0:
+            call("lt_q8_gemm_silu_quant_t", h, L["wgu_il_t"].t.vp, B.xq.vp, B.xd.vp, B.vq.vp, B.vd.vp, T, F, E)
+            vq, vd = B.vq.vp, B.vd.vp
+        else:
+            call("lt_q8_gemm_silu_t", h, L["wgu_il_t"].t.vp, B.xq.vp, B.xd.vp, B.v.vp, T, F, E)
+            vq, vd = B.xq.vp, B.xd.vp
+            call("lt_quant_q8_bm", h, B.v.vp, vq, vd, T, F)
+        call("lt_q8_gemm_t", h, L["wdown_t"].t.vp, vq, vd, None, B.xres.vp, B.x.vp, T, E, F)
 
 
 def forward_tokens(plan: DecodePlan, tokens, embeddings: np.ndarray | None = None) -> np.ndarray:

@@ -37,3 +37,25 @@ def test_default_kernel_equals_dynamic_walk(gpu, N, K, T, monkeypatch):
     assert np.array_equal(got, run())
     for t in (W, Wt, x, xq, xd, resid, y):
         t.free()
+
+
+@pytest.mark.parametrize("F,K,T", [(4864, 896, 129), (4864, 896, 509), (96, 1024, 512), (32, 32, 500)])
+def test_silu_with_quant_at_prompt_lengths(gpu, F, K, T):
+    """The fused SiLU quant a narrow prefill takes past the batch sizes of a decode step, against the
+    two launches."""
+    print(f"[gpu-case] silu quant F={F} K={K} T={T}", flush=True)
+    rng = np.random.default_rng(F + K + T)
+    W = dr.DevTensor.from_host(q8.quantize_rows((0.1 * rng.standard_normal((2 * F, K))).astype(np.float32)), gpu)
+    Wt = dr.DevTensor.empty((int(_lib.raw("lt_q8_tiles_bytes")(2 * F, K)),), np.uint8, gpu)
+    call("lt_q8_tiles", gpu.handle, W.vp, Wt.vp, 2 * F, K)
+    x = dr.DevTensor.from_host(rng.standard_normal((T, K)).astype(np.float32), gpu)
+    q = [dr.DevTensor.empty((T * n,), np.int8, gpu) for n in (K, F, F)]
+    d = [dr.DevTensor.empty((T * n // 32,), np.uint16, gpu) for n in (K, F, F)]
+    v = dr.DevTensor.empty((T, F), np.float32, gpu)
+    call("lt_quant_q8_bm", gpu.handle, x.vp, q[0].vp, d[0].vp, T, K)
+    call("lt_q8_gemm_silu_t", gpu.handle, Wt.vp, q[0].vp, d[0].vp, v.vp, T, F, K)
+    call("lt_quant_q8_bm", gpu.handle, v.vp, q[1].vp, d[1].vp, T, F)
+    call("lt_q8_gemm_silu_quant_t", gpu.handle, Wt.vp, q[0].vp, d[0].vp, q[2].vp, d[2].vp, T, F, K)
+    assert np.array_equal(q[1].to_host(), q[2].to_host()) and np.array_equal(d[1].to_host(), d[2].to_host())
+    for t in (W, Wt, x, v, *q, *d):
+        t.free()
