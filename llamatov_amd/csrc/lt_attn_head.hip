@@ -157,12 +157,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
       const int u = u0 + i;
       if (u >= nu) break;
       const int t0 = (w + NW * (u / NL)) * 64, ln = u % NL;
+      wave_fence();                                 // (the last line's reads, then this one's writes)
 #pragma unroll
       for (int j = 0; j < 8; j++) *(u32x4*)(kw + (8 * j + (l >> 3)) * kKRow + (l & 7) * 16) = kr[i][j];
       load_k(u + R, kr[i]);
-      if (kStep && Lnew >= t0 && Lnew < t0 + 64 && l < 8)   // the new row over its place
-        *(u32x4*)(kw + (Lnew - t0) * kKRow + l * 16) = *(const u32x4*)((const uint8_t*)sk + ln * 128 + l * 16);
-      asm volatile("" ::: "memory");
+      wave_fence();
+      if (kStep && Lnew >= t0 && Lnew < t0 + 64) {  // the new row over its place
+        if (l < 8)
+          *(u32x4*)(kw + (Lnew - t0) * kKRow + l * 16) = *(const u32x4*)((const uint8_t*)sk + ln * 128 + l * 16);
+        wave_fence();
+      }
       if (NL == 1 || ln == 0) acc = 0.0f;
 #pragma unroll
       for (int c = 0; c < 8; c++) {
@@ -249,11 +253,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
     };
     put_v(0, vr[0], 0);
     put_v(1, vr[1], RB);
+    wave_fence();
     read_block(0, 0, va[0], ea[0]);
     for (int p = 0; p < nv; p += D * RB) {
 #pragma unroll
       for (int j = 0; j < D; j++) {
         vr[j] = load_v(p + (j + D) * RB);
+        wave_fence();
         read_block((j + 1) & 1, p + (j + 1) * RB, va[(j + 1) & 1], ea[(j + 1) & 1]);
         put_v(j & 1, vr[(j + 2) % D], p + (j + 2) * RB);
 #pragma unroll
@@ -462,11 +468,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
     };
     put_v(0, vr[0], 0);
     put_v(1, vr[1], RB);
+    wave_fence();
     read_block(0, 0, va[0], ea[0]);
     for (int p = 0; p < n; p += D * RB) {
 #pragma unroll
       for (int j = 0; j < D; j++) {
         vr[j] = load_v(p + (j + D) * RB);
+        wave_fence();
         read_block((j + 1) & 1, p + (j + 1) * RB, va[(j + 1) & 1], ea[(j + 1) & 1]);
         put_v(j & 1, vr[(j + 2) % D], p + (j + 2) * RB);
 #pragma unroll

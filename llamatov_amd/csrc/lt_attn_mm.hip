@@ -292,12 +292,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
         const float* pb = P + n * ps + g4;
         const int cf = c1 < Lmin ? c1 : Lmin;       // every row attends the positions before cf
         int p = c0;
-        // block j of a group of D in buffer j % 2, written one block ahead of its folds
+        // block j of a group of D in buffer j % 2, written one block ahead of its folds; the fence
+        // keeps a block's folds behind its writes and before the next writes of its buffer
         put_v(0, vr[0]);
         for (; p + D * RB <= cf; p += D * RB) {
 #pragma unroll
           for (int j = 0; j < D; j++) {
             vr[j] = load_v(p + (j + D) * RB, RB);
+            wave_fence();
             put_v((j + 1) & 1, vr[(j + 1) % D]);
             const float* pj = pb + (p - c0) + j * RB;
 #pragma unroll
@@ -309,6 +311,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
 #pragma unroll
           for (int j = 0; j < D; j++) {
             vr[j] = load_v(p + (j + D) * RB, RB);
+            wave_fence();
             put_v((j + 1) & 1, vr[(j + 1) % D]);
             if (p + j * RB >= c1) continue;
             const float* pj = pb + (p - c0) + j * RB;
@@ -370,11 +373,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
     int Lq[QPW];
 #pragma unroll
     for (int u = 0; u < QPW; u++) Lq[u] = rowL(r0 + u);
-    auto wave_fence = [&]() {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     if (per <= 32) {
       const int hl = l & 31;
       for (int s = l >> 5; s < S; s += 2) {         // S is even
@@ -459,6 +457,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
         for (int j = 0; j < D; j++) {
           vr[j] = load_cur(cl);
           cl = next(cl);
+          wave_fence();
           put_v((j + 1) & 1, vr[(j + 1) % D]);
           if (cur.n > 0) {
             const int p = cur.s * per + cur.j, left = cur.n - cur.j;

@@ -372,6 +372,14 @@ __device__ __forceinline__ size_t q8_out_block(int obm, int nh, int hd, size_t g
   return (g - row * nbr) * (size_t)obm + row;
 }
 
+// Orders one wave's LDS accesses before it against those after it, for the compiler: the hardware
+// runs a wave's LDS instructions in order, so lanes of one wave hand data over with this alone.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- fp32 matrix instructions ----------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
