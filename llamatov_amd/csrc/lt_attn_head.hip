@@ -267,13 +267,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
 #pragma unroll
           for (int d = 0; d < DT; d++)
             o[d] = mma(va[j & 1][i][d], ea[j & 1][i], o[d]);
+        settle(o);
         if (p + (j + 1) * RB >= nv) break;          // (the rest of the group: zero rows)
       }
     }
   }
-  // the matrix results complete before what reads them in a later block (lt_attn_mm.hip)
-#pragma unroll
-  for (int d = 0; d < DT; d++) asm volatile("s_nop 10" : "+v"(o[d]));
   __syncthreads();                                  // Z
   if (w < NP && n16 == 0) {
     const float z = sm[NW];
@@ -359,34 +357,41 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
     for (int j = 0; j < NU; j++) kb[1][j] = load_unit((w + NW) * 16, j);
   }
 
+  // a tile's scores, its units replaced by those of the tile at `next` where there is one (a constant: a
+  // branch around the loads would cut the chain into several blocks)
+  auto s_tile = [&](u32x4 (&kt)[NU], int next, auto more) {
+    f32x4 s[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int j = 0; j < NU; j++) {
+      const u32x4 k = kt[j];
+      if (kF16) {
+        uint32_t r[4] = {__builtin_amdgcn_perm(k.z, k.x, 0x05040100u), __builtin_amdgcn_perm(k.z, k.x, 0x07060302u),
+                         __builtin_amdgcn_perm(k.w, k.y, 0x05040100u), __builtin_amdgcn_perm(k.w, k.y, 0x07060302u)};
+        if constexpr (decltype(more)::value) kt[j] = load_unit(next, j);
+        transpose4(r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          s[0] = mma(lt_h2f((uint16_t)(r[e] & 0xFFFFu)), qr[8 * j + 2 * e], s[0]);
+          s[0] = mma(lt_h2f((uint16_t)(r[e] >> 16)), qr[8 * j + 2 * e + 1], s[0]);
+        }
+      } else {
+        uint32_t r[4] = {k.x, k.y, k.z, k.w};
+        if constexpr (decltype(more)::value) kt[j] = load_unit(next, j);
+        transpose4(r);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[0] = mma(__uint_as_float(r[e]), qr[4 * j + e], s[0]);
+      }
+    }
+    settle(s);
+    return s[0];
+  };
   float mx = -1e30f;
   for (int p = w * 16; p < n; p += 32 * NW) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int pi = p + 16 * NW * i;
+      const int pi = p + 16 * NW * i, next = pi + 32 * NW;
       if (pi < n) {
-        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int j = 0; j < NU; j++) {
-          const u32x4 k = kb[i][j];
-          if (kF16) {
-            uint32_t r[4] = {__builtin_amdgcn_perm(k.z, k.x, 0x05040100u), __builtin_amdgcn_perm(k.z, k.x, 0x07060302u),
-                             __builtin_amdgcn_perm(k.w, k.y, 0x05040100u), __builtin_amdgcn_perm(k.w, k.y, 0x07060302u)};
-            if (pi + 32 * NW < n) kb[i][j] = load_unit(pi + 32 * NW, j);
-            transpose4(r);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-              s = mma(lt_h2f((uint16_t)(r[e] & 0xFFFFu)), qr[8 * j + 2 * e], s);
-              s = mma(lt_h2f((uint16_t)(r[e] >> 16)), qr[8 * j + 2 * e + 1], s);
-            }
-          } else {
-            uint32_t r[4] = {k.x, k.y, k.z, k.w};
-            if (pi + 32 * NW < n) kb[i][j] = load_unit(pi + 32 * NW, j);
-            transpose4(r);
-#pragma unroll
-            for (int e = 0; e < 4; e++) s = mma(__uint_as_float(r[e]), qr[4 * j + e], s);
-          }
-        }
+        f32x4 s = next < n ? s_tile(kb[i], next, std::true_type{}) : s_tile(kb[i], next, std::false_type{});
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           s[r] = s[r] * A.scale;
@@ -479,12 +484,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
         put_v(j & 1, vr[(j + 2) % D], p + (j + 2) * RB);
 #pragma unroll
         for (int i = 0; i < NS; i++) o[0] = mma(va[j & 1][i], ea[j & 1][i], o[0]);
+        settle(o);
         if (p + (j + 1) * RB >= n) break;           // (the rest of the group: zero rows)
       }
     }
   }
-  // the matrix results complete before what reads them in a later block (lt_attn_mm.hip)
-  asm volatile("s_nop 10" : "+v"(o[0]));
   __syncthreads();                                  // the exps are free
   float* so = P;                                    // [rep][HD]
   if (w < NP && n16 < rep) {

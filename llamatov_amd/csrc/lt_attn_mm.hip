@@ -236,12 +236,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
     return (not_finite_bits(x.x, kF16) | not_finite_bits(x.y, kF16) | not_finite_bits(x.z, kF16) |
             not_finite_bits(x.w, kF16)) != 0;
   };
-  // the matrix results complete before whatever reads them next (the compiler's own waits do
-  // not reach a register copy in a later block: seen in this kernel's assembly)
-  auto settle = [&]() {
-    if constexpr (DT == 2) asm volatile("s_nop 10" : "+v"(o[0]), "+v"(o[DT - 1]));
-    else asm volatile("s_nop 10" : "+v"(o[0]));
-  };
 
   if constexpr (!kSplit) {
     const bool multi = Lmax > A.cap;
@@ -305,8 +299,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
 #pragma unroll
             for (int i = 0; i < RB / 4; i++) fold(j & 1, i, pj[4 * i]);
           }
+          settle(o);
         }
-        settle();
         for (; p < c1; p += D * RB) {               // the rows' last positions
 #pragma unroll
           for (int j = 0; j < D; j++) {
@@ -321,7 +315,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
 #pragma unroll
               for (int i = 0; i < RB / 4; i++) fold(j & 1, i, pj[4 * i]);
             }
-            settle();
+            settle(o);
           }
         }
       }
@@ -474,7 +468,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
                 fold(j & 1, i + 1, 4 * i + 4 + g4 < left ? b1 : 0.0f);
               }
             }
-            settle();
+            settle(o);
             if (cur.j + RB >= cur.n) {                // the split's last block
               const float ws = ssm[n * S + cur.s];
 #pragma unroll

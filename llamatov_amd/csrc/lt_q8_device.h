@@ -390,6 +390,16 @@ __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// The matrix results in o complete before whatever reads them in a later basic block: the compiler's own
+// waits do not reach a register copy there (seen in the assembly of lt_attn_mm.hip), so a chain is
+// settled in the block of its last instruction, before any branch.
+template <int N>
+__device__ __forceinline__ void settle(f32x4 (&o)[N]) {
+  static_assert(N == 1 || N == 2, "settle: one or two accumulators");
+  if constexpr (N == 2) asm volatile("s_nop 10" : "+v"(o[0]), "+v"(o[1]));
+  else asm volatile("s_nop 10" : "+v"(o[0]));
+}
+
 // 4 x 4 transpose of four registers over the four 16-lane groups: group g's register r becomes
 // group r's register g.
 __device__ __forceinline__ void transpose4(uint32_t (&r)[4]) {
