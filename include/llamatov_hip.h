@@ -589,6 +589,14 @@ LT_API int lt_sample(lt_ctx* ctx, const float* logits, int V, lt_sample_params* 
  * (k + 1/2) * dq for |k| <= 140).  Synchronous; 0 or an error code. */
 LT_API int lt_selftest_numerics(lt_ctx* ctx, unsigned long long* out);
 
+/* The same for what the attention kernels' bit-identity rests on; 3 counters: out[0] = binary32
+ * patterns (all 2^32) whose exponential by lt_expf_n, several values at once, differs in any bit
+ * from lt_expf_sel, out[1] = sums of 512 products on the fp32 matrix instruction that differ from
+ * the fmaf chain in ascending order (operands near 1, over 2^-126 .. 2^63, subnormal, with
+ * underflowing products, with cancelling pairs, and with zeros, infinities and nans), out[2] =
+ * sums tried.  Synchronous; 0 or an error code. */
+LT_API int lt_selftest_attn_numerics(lt_ctx* ctx, unsigned long long* out);
+
 /* ---- graphs (replaces cuStreamBeginCapture/EndCapture/GraphInstantiate/GraphLaunch,
  *      GraphRunner.capture / replay, bpd/lib/dev_residency.py:1732-1818) ---- */
 LT_API int lt_graph_begin(lt_ctx* ctx);

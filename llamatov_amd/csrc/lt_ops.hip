@@ -495,6 +495,80 @@ __global__ __launch_bounds__(256) void k_check_quotient(unsigned long long* out)
   atomicAdd(&out[2], cases);
 }
 
+// Every binary32 pattern: lt_expf_n, in each width the attention kernels use, against lt_expf_sel.
+__global__ __launch_bounds__(256) void k_check_expf_n(unsigned long long* bad) {
+  unsigned long long n = 0;
+  const uint64_t stride = (uint64_t)gridDim.x * 1024u;
+  for (uint64_t u = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u; u < (1ull << 32); u += stride) {
+    float x[4], want[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      x[i] = __builtin_bit_cast(float, (uint32_t)u + (uint32_t)i);
+      want[i] = lt_expf_sel(x[i]);
+    }
+    float a[2] = {x[0], x[1]}, b[2] = {x[2], x[3]}, c[1] = {x[1]};
+    lt_expf_n(x);
+    lt_expf_n(a);
+    lt_expf_n(b);
+    lt_expf_n(c);
+    const float got[4] = {a[0], a[1], b[0], b[1]};
+    auto differ = [](float p, float q) { return __builtin_bit_cast(uint32_t, p) != __builtin_bit_cast(uint32_t, q); };
+#pragma unroll
+    for (int i = 0; i < 4; i++) n += (differ(x[i], want[i]) || differ(got[i], want[i])) ? 1u : 0u;
+    n += differ(c[0], want[1]) ? 1u : 0u;
+  }
+  if (n) atomicAdd(bad, n);
+}
+
+// One operand of a matrix chain: class 0 binary orders near 1; 1 over 2^-126 .. 2^63; 2 the A side
+// subnormal; 3 products about and below the smallest subnormal; 4 each product after the first of a
+// pair cancels it but for the last bits; 5 as 1 with zeros of both signs, infinities and nans.
+__device__ float chain_operand(int cls, uint32_t wg, bool is_b, int i, int k) {
+  const int kk = cls == 4 ? k & ~1 : k;
+  uint32_t h = (wg * 2u + (is_b ? 1u : 0u)) * 0x9E3779B1u + (uint32_t)(i * 4096 + kk) * 0x85EBCA77u;
+  h ^= h >> 15; h *= 0x2C1B3C6Du; h ^= h >> 12; h *= 0x297A2D39u; h ^= h >> 15;
+  const uint32_t e = h >> 9 & 0xFFu, sm = (h & 0x800001FFu) | (h * 0x9E3779B1u >> 9 & 0x7FFE00u);
+  uint32_t ex;                                      // the biased exponent
+  switch (cls) {
+    case 0: ex = 123u + (e & 7u); break;
+    case 2: ex = is_b ? 100u + e % 56u : 0u; break;
+    case 3: ex = is_b ? 90u + e % 21u : 1u + e % 30u; break;
+    case 4: ex = 126u; break;
+    default: ex = 1u + e % 190u; break;
+  }
+  uint32_t u = sm | ex << 23;
+  if (cls == 4 && (k & 1)) u = is_b ? u ^ 0x80000000u : u ^ 1u;
+  if (cls == 5 && (h >> 5) % 67u == 0) {
+    const uint32_t s[4] = {0u, 0x80000000u, 0x7F800000u | (h & 0x80000000u), 0x7FC00000u};
+    u = s[(h >> 3) % 29u == 0 ? 2u + (h & 1u) : h & 1u];
+  }
+  return __builtin_bit_cast(float, u);
+}
+
+// One wave per workgroup: 256 chains of 512 terms on v_mfma_f32_16x16x4_f32 (mma, lt_q8_device.h)
+// against fmaf in ascending order, every bit (two nans agree).
+__global__ __launch_bounds__(64) void k_check_chain(unsigned long long* out) {
+  constexpr int kTerms = 512;
+  const int l = threadIdx.x, n = l & 15, g = l >> 4;
+  const uint32_t wg = blockIdx.x;
+  const int cls = (int)(wg % 6u);
+  f32x4 acc[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
+  for (int k = 0; k < kTerms; k += 4) {
+    acc[0] = mma(chain_operand(cls, wg, false, n, k + g), chain_operand(cls, wg, true, n, k + g), acc[0]);
+    settle(acc);
+  }
+  unsigned long long bad = 0;
+  for (int r = 0; r < 4; r++) {
+    float want = 0.0f;
+    for (int k = 0; k < kTerms; k++)
+      want = fmaf(chain_operand(cls, wg, false, 4 * g + r, k), chain_operand(cls, wg, true, n, k), want);
+    const float got = acc[0][r];
+    if (__builtin_bit_cast(uint32_t, got) != __builtin_bit_cast(uint32_t, want) && !(got != got && want != want)) bad++;
+  }
+  if (bad) atomicAdd(&out[0], bad);
+  atomicAdd(&out[1], 4ull);
+}
+
 // Repack a Q8_0 matrix [N][nb] (34-byte blocks) into the planar layout (lt_q8_device.h):
 // thread per block; its 32 quants go to the two 16-byte halves of its item slot, its scale to
 // the scale plane.  Byte loads: the source blocks are only 2-byte aligned.
@@ -729,6 +803,26 @@ int lt_selftest_numerics(lt_ctx* ctx, unsigned long long* out) {
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   hipFree(d);
   if (e != hipSuccess) return lt_fail_hip(e, "lt_selftest_numerics", __FILE__, __LINE__);
+  return LT_OK;
+}
+
+int lt_selftest_attn_numerics(lt_ctx* ctx, unsigned long long* out) {
+  LT_REQUIRE(ctx && out, "lt_selftest_attn_numerics: null argument");
+  unsigned long long* d = nullptr;
+  LT_CHECK(hipMalloc(&d, 3 * sizeof(unsigned long long)));
+  hipError_t e = hipMemsetAsync(d, 0, 3 * sizeof(unsigned long long), ctx->stream);
+  if (e == hipSuccess) {
+    k_check_expf_n<<<4096, 256, 0, ctx->stream>>>(d);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) {
+    k_check_chain<<<1536, 64, 0, ctx->stream>>>(d + 1);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(out, d, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  hipFree(d);
+  if (e != hipSuccess) return lt_fail_hip(e, "lt_selftest_attn_numerics", __FILE__, __LINE__);
   return LT_OK;
 }
 

@@ -1,7 +1,8 @@
 """The engine quantizer's division-free quotient (lt_numerics.h: lt_q8_quotient, used by
 every device quantizer) equals IEEE division x / dq bit for bit, on the CPU over every
 positive finite fp16 scale (tests/csrc/q8_quotient_check.c), and on the device together
-with the hardware fp16 conversion of the scale (lt_selftest_numerics)."""
+with the hardware fp16 conversion of the scale (lt_selftest_numerics); and the exponentials and matrix
+chains of the attention kernels (lt_selftest_attn_numerics)."""
 import ctypes
 import shutil
 import subprocess
@@ -67,3 +68,16 @@ def test_device_fp16_conversion_and_quotient(gpu):
     f2h_bad, q_bits, q_bad, cases = list(out)
     assert cases > 8_000_000
     assert (f2h_bad, q_bits, q_bad) == (0, 0, 0)
+
+
+@pytest.mark.gpu
+def test_device_exponentials_and_matrix_chains(gpu):
+    """What the attention kernels' bit-identity rests on: lt_expf_n is lt_expf_sel on every binary32
+    input, and v_mfma_f32_16x16x4_f32 is a chain of four fmas in ascending order, each with one
+    rounding, over subnormal, wide-range, underflowing, cancelling and special operands too."""
+    from llamatov_amd import _lib
+    out = (ctypes.c_ulonglong * 3)()
+    _lib.call("lt_selftest_attn_numerics", gpu.handle, out)
+    expf_bad, chain_bad, chains = list(out)
+    assert chains == 1536 * 256
+    assert (expf_bad, chain_bad) == (0, 0)
