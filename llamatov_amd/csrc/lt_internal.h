@@ -103,6 +103,8 @@ struct LtAttnHead {
   int batch, nh, nkv;
   float scale;
   int maxt;
+  int rep;         // set by the launcher: nh / nkv
+  uint32_t rnkv;   // set by the launcher: for pair / nkv
 };
 bool lt_attn_head_covers(const lt_ctx* ctx, int batch, int nh, int nkv, int hd, int maxt, bool step);
 int lt_attn_head(lt_ctx* ctx, LtAttnHead A, int hd, bool f16, bool step);

@@ -390,6 +390,15 @@ __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// The maximum over lanes n16, n16 + 16, n16 + 32, n16 + 48 (order-free), in each of them.
+__device__ __forceinline__ float max_over_groups(float a) {
+  const uint32_t u = __float_as_uint(a);
+  const u32x2 x = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t v = __float_as_uint(fmaxf(__uint_as_float(x.x), __uint_as_float(x.y)));
+  const u32x2 y = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return fmaxf(__uint_as_float(y.x), __uint_as_float(y.y));
+}
+
 // The matrix results in o complete before whatever reads them in a later basic block: the compiler's own
 // waits do not reach a register copy there (seen in the assembly of lt_attn_mm.hip), so a chain is
 // settled in the block of its last instruction, before any branch.

@@ -16,6 +16,8 @@ from llamatov_amd._lib import LT_KV_F16, LT_KV_F32, call
 pytestmark = pytest.mark.gpu
 
 LENS = (1, 15, 16, 17, 31, 33, 64, 65, 255, 256, 257, 511, 513, 1024, 1025, 1290)
+# exps one, two or four at a time; one position a thread or more
+EXP_LENS = (63, 127, 128, 129, 192, 193, 320, 321, 384, 385, 449, 512)
 
 
 def _cache(rng, shape, f16):
@@ -26,6 +28,16 @@ def _cache(rng, shape, f16):
 @pytest.mark.parametrize("kv_dtype", [LT_KV_F32, LT_KV_F16])
 @pytest.mark.parametrize("nh,nkv,hd", [(2, 1, 64), (3, 3, 128)])
 def test_step_lengths(gpu, oracle, kv_dtype, nh, nkv, hd):
+    _step(gpu, oracle, kv_dtype, nh, nkv, hd, LENS)
+
+
+@pytest.mark.parametrize("kv_dtype", [LT_KV_F32, LT_KV_F16])
+@pytest.mark.parametrize("nh,nkv,hd", [(2, 1, 64), (7, 7, 128)])
+def test_step_exps(gpu, oracle, kv_dtype, nh, nkv, hd):
+    _step(gpu, oracle, kv_dtype, nh, nkv, hd, EXP_LENS)
+
+
+def _step(gpu, oracle, kv_dtype, nh, nkv, hd, lens):
     f16, maxt, theta = kv_dtype == LT_KV_F16, 1300, 1e6
     rng = np.random.default_rng(hd)
     width, scale = nkv * hd, float(hd ** -0.5)
@@ -33,7 +45,7 @@ def test_step_lengths(gpu, oracle, kv_dtype, nh, nkv, hd):
     freqs = up(oracle.rope_freqs(hd, theta))
     base_k, base_v = _cache(rng, (maxt, width), f16), _cache(rng, (maxt, width), f16)
     nan = 0x7E00 if f16 else np.nan
-    for L in (0,) + tuple(n - 1 for n in LENS[1:]) + (maxt - 1,):
+    for L in (0,) + tuple(n - 1 for n in lens[1:]) + (maxt - 1,):
         print(f"[gpu-case] attn head step nh={nh} hd={hd} f16={f16} L={L}", flush=True)
         kc, vc = base_k.copy(), base_v.copy()
         kc[L:], vc[L:] = nan, nan
@@ -59,11 +71,22 @@ def test_step_lengths(gpu, oracle, kv_dtype, nh, nkv, hd):
 @pytest.mark.parametrize("nh,nkv,hd,B", [(14, 2, 64, 16), (4, 1, 128, 16), (64, 8, 64, 4), (64, 8, 64, 5),
                                           (14, 2, 64, 20), (32, 2, 128, 10), (8, 4, 64, 40), (80, 80, 64, 4), (51, 3, 64, 6)])
 def test_batched_lengths(gpu, oracle, kv_dtype, nh, nkv, hd, B):
+    _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, LENS)
+
+
+# (odd counts of KV groups, of (sequence, group) pairs and of both, per head and per group)
+@pytest.mark.parametrize("kv_dtype", [LT_KV_F32, LT_KV_F16])
+@pytest.mark.parametrize("nh,nkv,hd,B", [(6, 3, 64, 23), (7, 7, 128, 30), (1, 1, 64, 25), (32, 8, 128, 15), (21, 3, 64, 25)])
+def test_batched_exps(gpu, oracle, kv_dtype, nh, nkv, hd, B):
+    _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, EXP_LENS + (1, 2))
+
+
+def _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, all_lens):
     f16, maxt = kv_dtype == LT_KV_F16, 1300
     rng = np.random.default_rng(B * hd)
     width, scale = nkv * hd, float(hd ** -0.5)
     up = lambda a: dr.DevTensor.from_host(a, gpu)
-    lens = [LENS[(5 * b + 3) % len(LENS)] for b in range(B)]
+    lens = [all_lens[(5 * b + 3) % len(all_lens)] for b in range(B)]
     print(f"[gpu-case] attn head batch nh={nh} hd={hd} f16={f16} B={B} lens={lens}", flush=True)
     k, v = _cache(rng, (B, maxt, width), f16), _cache(rng, (B, maxt, width), f16)
     for b, L in enumerate(lens):
