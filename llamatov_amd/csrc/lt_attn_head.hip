@@ -237,7 +237,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4,
   const int n_up = (nv + D * RB - 1) / (D * RB) * (D * RB);
   const int n_all = n_up > n ? n_up : n;
   if (n_all <= 64 * NW) {                           // one position a thread
-    float e[1] = {P[e_slot(tid)] - m};
+    float e[1] = {P[e_slot(tid < n_all ? tid : 0)] - m};   // (the exps' LDS may end at n_all)
     lt_expf_n(e);
     if (tid < n_all) P[e_slot(tid)] = tid < n ? e[0] : 0.0f;
   } else {

@@ -37,8 +37,17 @@ def test_step_exps(gpu, oracle, kv_dtype, nh, nkv, hd):
     _step(gpu, oracle, kv_dtype, nh, nkv, hd, EXP_LENS)
 
 
-def _step(gpu, oracle, kv_dtype, nh, nkv, hd, lens):
-    f16, maxt, theta = kv_dtype == LT_KV_F16, 1300, 1e6
+# (less LDS for the exps than threads: only the context's own are read)
+@pytest.mark.parametrize("kv_dtype", [LT_KV_F32, LT_KV_F16])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("maxt", [1, 20, 256, 300])
+def test_small_caches(gpu, oracle, kv_dtype, hd, maxt):
+    _step(gpu, oracle, kv_dtype, 2, 1, hd, (1, min(maxt, 17)), maxt)
+    _batched(gpu, oracle, kv_dtype, 2, 1, hd, 3, (1, maxt, min(maxt, 17)), maxt)
+
+
+def _step(gpu, oracle, kv_dtype, nh, nkv, hd, lens, maxt=1300):
+    f16, theta = kv_dtype == LT_KV_F16, 1e6
     rng = np.random.default_rng(hd)
     width, scale = nkv * hd, float(hd ** -0.5)
     up = lambda a: dr.DevTensor.from_host(a, gpu)
@@ -81,8 +90,8 @@ def test_batched_exps(gpu, oracle, kv_dtype, nh, nkv, hd, B):
     _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, EXP_LENS + (1, 2))
 
 
-def _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, all_lens):
-    f16, maxt = kv_dtype == LT_KV_F16, 1300
+def _batched(gpu, oracle, kv_dtype, nh, nkv, hd, B, all_lens, maxt=1300):
+    f16 = kv_dtype == LT_KV_F16
     rng = np.random.default_rng(B * hd)
     width, scale = nkv * hd, float(hd ** -0.5)
     up = lambda a: dr.DevTensor.from_host(a, gpu)
