@@ -383,6 +383,9 @@ LT_API int lt_rmsnorm_quant_bm(lt_ctx* ctx, const float* x, const float* w, int8
  * bits with far fewer cache lines touched per block.  The tile copy must be below 2 GiB. */
 LT_API int lt_q8_gemm_t(lt_ctx* ctx, const void* Wt, const int8_t* Xq, const uint16_t* Xd, const float* bias,
                         const float* resid, float* Y, int T, int N, int K);
+/* The kernel lt_q8_gemm_t takes for a product on a device of num_cus CUs: 0 .. 2 the 128-token kernel with its
+ * dynamic / 2-slot / 4-slot walk of K, 3 the leaf-split kernel, -1 for sizes it refuses.  All give the same bits. */
+LT_API int lt_q8_gemm_t_kernel(int num_cus, int T, int N, int K);
 LT_API int lt_q8_gemm_silu_t(lt_ctx* ctx, const void* Wgut, const int8_t* Xq, const uint16_t* Xd, float* V, int T,
                              int F, int K);
 /* lt_q8_gemm_silu_t followed by lt_quant_q8_bm of its output, in one launch (no fp32 output):

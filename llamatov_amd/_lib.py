@@ -108,6 +108,7 @@ _SIGS = {
     "lt_quant_q8_bm": (c_int, [_P, _P, _P, _P, c_int, c_int]),
     "lt_rmsnorm_quant_bm": (c_int, [_P, _P, _P, _P, _P, c_int, c_int, c_float]),
     "lt_q8_gemm_t": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int]),
+    "lt_q8_gemm_t_kernel": (c_int, [c_int, c_int, c_int, c_int]),
     "lt_q8_gemm_silu_t": (c_int, [_P, _P, _P, _P, _P, c_int, c_int, c_int]),
     "lt_q8_gemm_silu_quant_t": (c_int, [_P, _P, _P, _P, _P, _P, c_int, c_int, c_int]),
     "lt_q8_tiles_rope": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, c_int]),

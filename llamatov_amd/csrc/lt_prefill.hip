@@ -1086,29 +1086,64 @@ int check_gemm(const char* fn, const void* W, const int8_t* Xq, const uint16_t* 
   return LT_OK;
 }
 
-// Which tiled launches take the leaf-split kernel (LT_GEMM_LS=0 / 1 forces k_q8_gemm / the
-// leaf-split kernel, read at every launch).  k_q8_gemm's tiles are 128 tokens, one 32 x 32 tile a
-// wave, with the fewest instructions where K % 2048 == 0 lets its leaves go in static groups; the
-// leaf-split kernel's are 32 tokens, 4 to 16 waves a tile, its schedule fixed at compile time up to
-// 5 blocks a leaf.  Measured per launch over rotated weight copies, k_q8_gemm / leaf-split (us):
-//  - one block per leaf (K <= 1024), any size: k_q8_gemm walks run-time leaves of one block there:
-//    9728 x 896 at T = 256 / 509 / 2048 24.5 / 15.6, 40.9 / 25.6, 134 / 84.8; 151936 x 896 at 128
-//    and 256 137 / 85, 281 / 198; 1152 x 896 at 2048 27.1 / 15.9;
-//  - two (K <= 2048): unless the grouped walk applies and has 3 waves per SIMD: 11008 x 2048 at 256
-//    and 512 27.4 / 28.9, 46.8 / 51.1; 2048 x 2048 at 512 18.7 / 14.7;
-//  - three to five (K <= 5120): up to 128 tokens and while k_q8_gemm's grid holds less than 2
-//    workgroups per CU: 28672 x 4096 at 32 / 64 / 128 / 256 61 / 33, 63 / 44, 69 / 71, 116 / 127;
-//    6144 x 4096 at 256 / 400 33.9 / 32.4, 41.9 / 47.0; 4096 x 4096 at 256 / 512 29.7 / 23.0, 36.2 /
-//    40.2; 896 x 4864 at 509 and 1024 41.7 / 11.9, 46 / 26.9;
-//  - more: up to 64 tokens or on the same grids: 4096 x 14336 at 64 / 256 / 400 / 512 95 / 24.7, 95 /
-//    71, 107 / 103, 109 / 118.
-bool take_ls(const lt_ctx* ctx, const GemmParams& P) {
-  const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+// How k_q8_gemm walks a tiled launch: 0 the dynamic walk; where K is a multiple of 2048 (an even number of
+// blocks per leaf, bpl) also leaves in static groups, 1 with a 2-slot ring, 2 (bpl % 4 == 0) with a 4-slot
+// ring and pipelined MFMAs.  A CU holds three workgroups of walk 1 and two of walk 2, whose round takes about
+// 0.8 of the former's time, so the rounds of workgroups decide (2-slot / 4-slot, us over cold weights:
+// 4096 x 4096 at 512, 640 and 1024 tokens 41.1 / 36.3, 45.2 / 59.7, 81.1 / 68.4; 6144 x 4096 at 320 and 512
+// 44.0 / 59.6, 46.2 / 61.6; 28672 x 4096 at 128 and 512 90.6 / 78.5, 218 / 237).  Other bpl: 2 blocks a leaf
+// always in groups (dynamic / 2-slot: 11008 x 2048 at 64 / 256 / 512 29.8 / 24.3, 37.6 / 29.2, 71.9 / 54.8), 6
+// where the launch fills the chip, more never (4096 x 14336 at 512 113.5 / 120.2).
+// LT_GEMM_GROUPED=0 / 1 / 2 forces a walk where K allows it (read at every launch).
+struct GemmWalk {
+  int walk;
+  long rounds;   // of resident workgroups
+};
+GemmWalk gemm_walk(long cus, const GemmParams& P) {
   const long wgs = (long)((P.nrt + 7) / 8) * 8 * ((P.T + kGemmTokens - 1) / kGemmTokens);
+  const long r3 = (wgs + 3 * cus - 1) / (3 * cus), r2 = (wgs + 2 * cus - 1) / (2 * cus);
+  const int bpl = P.K / 1024;
+  int walk = 0;
+  if (P.K % 2048 == 0) {
+    const long waves = (long)P.nrt * ((P.T + 31) / 32);
+    const char* force = getenv("LT_GEMM_GROUPED");
+    if (force) walk = atoi(force);
+    else if (bpl % 4 == 0) walk = 4 * r2 < 5 * r3 ? 2 : 1;
+    else walk = bpl == 2 || (bpl <= 8 && waves >= 12 * cus) ? 1 : 0;
+    if (walk < 0 || walk > 2 || (walk == 2 && bpl % 4 != 0)) walk = 0;
+  }
+  return GemmWalk{walk, walk == 2 ? r2 : r3};
+}
+
+// Which tiled launches take the leaf-split kernel (LT_GEMM_LS=0 / 1 forces k_q8_gemm / the leaf-split kernel,
+// read at every launch).  k_q8_gemm's tiles are 128 tokens, one 32 x 32 tile a wave, and its time goes by
+// rounds of resident workgroups; the leaf-split kernel's are 32 tokens, 4 to 16 waves a tile, its schedule
+// fixed at compile time up to 5 blocks a leaf, and its time goes by tiles.  Per launch, k_q8_gemm / leaf-split
+// as launched by default (us over cold weights; tiles per CU in brackets):
+//  - one block per leaf (K <= 1024), any size: 9728 x 896 at T = 64 / 512 / 2048 20.5 / 7.6, 46.7 / 30.3,
+//    152 / 101; 1152 x 896 at 2048 26.6 / 16.2;
+//  - two, in groups: below 6.5 tiles per CU and round: 11008 x 2048 at 128 (5.4, one round) 25.8 / 21.2, 192
+//    (8.1) 28.5 / 29.3, 256 (10.8) 29.2 / 37.7, 280 (12.1, two rounds) 48.4 / 41.0, 384 (16) 50.3 / 53.7;
+//    4096 x 2048 at 256 (4) 21.1 / 17.3, 400 (6.5) 22.8 / 24.0;
+//  - two, not in groups: below 10: 8960 x 1536 at 128 (4.4) / 768 (26, three rounds) / 1024 (35) 26.6 / 18.1,
+//    78 / 75, 91.4 / 98.1; 1536 x 1536 at 1024 (6) / 2048 (12) 25.3 / 17.6, 32.7 / 35.1;
+//  - three to five: up to 128 tokens, and below 7 on the 4-slot walk, 9 on the dynamic walk of at most four, else
+//    8: 28672 x 4096 at 64 / 128 71.7 / 47.1, 78.5 / 76.7, 160 (18, three rounds) 126 / 90, 256 (28) 130 / 135;
+//    4096 x 4096 at 400 (6.5) 35.0 / 34.4, 512 (8) 36.1 / 40.1; 6144 x 4096 at 320 (7.5) 43.7 / 38.4, 400 (9.8)
+//    44.7 / 47.9; 896 x 4864 at 512 (2) / 2048 (8) 41.8 / 14.7, 47.7 / 51.2; 3584 x 3584 at 640 (8.75) 48.2 /
+//    39.2, 672 (9) 48.2 / 40.2, 1024 (14, two rounds) 75 / 64, but 18944 x 3584 at 256 (18.5, two) 87.6 / 89.1
+//    and 512 (37, four) 159 / 165;
+//  - more: up to 64 tokens, and below 8 or 7 tiles per CU: 4096 x 14336 at 64 / 256 94.8 / 24.2, 96 / 68, 448
+//    (7) 112 / 106, 512 (8) 113 / 115; 8192 x 8192 at 128 (4) / 256 (8) 53.8 / 47.1, 66 / 75; 16384 x 8192 at
+//    64 (4) / 128 (8) 66.8 / 52.9, 74 / 83.
+bool take_ls(long cus, const GemmParams& P) {
   const int bpl = (P.K / 32 + 31) / 32;             // blocks per leaf
-  if (bpl == 1) return true;
-  if (bpl == 2) return !(P.K % 2048 == 0 && (long)P.nrt * ((P.T + 31) / 32) >= 12 * cus);
-  return P.T <= (bpl <= 5 ? 128 : 64) || wgs < 2 * cus;
+  if (bpl == 1 || (bpl > 2 && P.T <= (bpl <= 5 ? 128 : 64))) return true;
+  const GemmWalk w = gemm_walk(cus, P);
+  const long tiles = (long)((P.nrt + 7) / 8) * 8 * ((P.T + 31) / 32);
+  if (bpl > 5) return tiles < (w.walk == 2 ? 7 : 8) * cus;
+  const long halves = bpl == 2 ? (w.walk ? 13 : 20) : w.walk == 2 ? 14 : w.walk == 0 && bpl <= 4 ? 18 : 16;
+  return 2 * tiles < halves * cus * w.rounds;
 }
 int ls_mode() {
   const char* s = getenv("LT_GEMM_LS");
@@ -1143,20 +1178,20 @@ void launch_ls(lt_ctx* ctx, const GemmParams& P, unsigned grid) {
 template <GemmEpi EPI, bool kTiled>
 int launch_gemm(lt_ctx* ctx, GemmParams P) {
   P.nrt = (P.N + 31) / 32;
+  const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   if constexpr (kTiled) {
     const int mode = ls_mode();
-    if (mode == 1 || (mode < 0 && take_ls(ctx, P))) {
+    if (mode == 1 || (mode < 0 && take_ls(cus, P))) {
       P.ntt = (P.T + 31) / 32;
       const long gls = (long)((P.nrt + 7) / 8) * 8 * P.ntt;
-      // Waves per tile (LT_GEMM_LS_W=4 / 8 / 16 forces one, read at every launch).  At most one
-      // tile per CU: 8, and 16 when each leaf holds 3 to 5 blocks (T = 64, 8 / 16 waves: 896 x
-      // 4864 7.95 / 7.58 us, 4096 x 4096 9.52 / 9.12, 896 x 896 4.19 / 4.26).  More tiles: 4,
-      // but 8 where that is what fits the compile-time schedule, 3 to 5 blocks (4 / 8 waves:
-      // 896 x 4864 at T = 509 17.8 / 12.9, 6144 x 4096 at 64 and 256 14.4 / 10.4, 33.9 / 25.0, 28672
-      // x 4096 at 64 38.3 / 30.8; one block: 9728 x 896 at 509 24.8 / 30.2).
+      // Waves per tile (LT_GEMM_LS_W=4 / 8 / 16 forces one, read at every launch).  At most one tile per CU:
+      // 8, and 16 when each leaf holds 3 to 5 blocks (T = 64, 8 / 16 waves, us: 896 x 4864 10.6 / 10.1, 4096
+      // x 4096 10.0 / 9.7, but 9728 x 896 8.8 / 8.5, 2048 x 2048 6.7 / 6.4).  More tiles: 4, but 8 where that
+      // is what fits the compile-time schedule, 3 to 5 blocks (4 / 8 waves: 896 x 4864 at T = 509 17.4 / 14.8,
+      // 6144 x 4096 at 64 and 256 16.4 / 15.0, 36.5 / 32.9, 28672 x 4096 at 64 50.8 / 47.1; one block: 9728 x
+      // 896 at 512 30.2 / 40.9).
       const char* wenv = getenv("LT_GEMM_LS_W");
       const int wforce = wenv ? atoi(wenv) : 0;
-      const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
       const int bpl = (P.K / 32 + 31) / 32;
       const bool mid = bpl >= 3 && bpl <= 5;
       const int w = wforce ? wforce : gls > cus ? (mid ? 8 : 4) : mid ? 16 : 8;
@@ -1169,33 +1204,10 @@ int launch_gemm(lt_ctx* ctx, GemmParams P) {
   P.ntt = (P.T + kGemmTokens - 1) / kGemmTokens;
   const long grid = (long)((P.nrt + 7) / 8) * 8 * P.ntt;
   if constexpr (kTiled) {
-    // K a multiple of 2048 (an even number of blocks per leaf, bpl): grouped leaves.  The 2-slot
-    // ring keeps 3 waves per SIMD (the other waves hide the latency), the 4-slot ring with
-    // pipelined MFMAs 2 (bpl % 4 == 0): a resident round of the latter takes about 0.8 of the
-    // former's time, so the rounds decide (2-slot / 4-slot, us: 4096 x 4096 at 512 and 1024 tokens
-    // 41.2 / 36.2, 80.3 / 68.2; 6144 x 4096 at 400 and 512 41.9 / 54.0, 44.2 / 55.8; 28672 x 4096 at
-    // 128 / 512 81 / 69, 203 / 215).  Other bpl: the 2-slot ring where it fills the chip, but not
-    // past 8 blocks a leaf (4096 x 14336 at 512 and 1024, dynamic / 2-slot 109 / 119, 220 / 239).
-    // LT_GEMM_GROUPED=0 / 1 / 2 forces the dynamic walk / the 2-slot / the 4-slot walk where
-    // K allows it (read at every launch).
-    if (P.K % 2048 == 0) {
-      const int bpl = P.K / 1024;
-      const long waves = (long)P.nrt * ((P.T + 31) / 32);
-      const long cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-      const long r2 = (waves + 12 * cus - 1) / (12 * cus), r4 = (waves + 8 * cus - 1) / (8 * cus);
-      const char* force = getenv("LT_GEMM_GROUPED");
-      const int walk = force                ? atoi(force)
-                       : bpl % 4 == 0       ? (4 * r4 < 5 * r2 ? 2 : 1)
-                       : bpl <= 8 && waves >= 12 * cus ? 1 : 0;
-      if (walk == 1) {
-        k_q8_gemm<EPI, true, 1><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
-        return lt_check_launch("k_q8_gemm");
-      }
-      if (walk == 2 && bpl % 4 == 0) {
-        k_q8_gemm<EPI, true, 2><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
-        return lt_check_launch("k_q8_gemm");
-      }
-    }
+    const int walk = gemm_walk(cus, P).walk;
+    if (walk == 1) k_q8_gemm<EPI, true, 1><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
+    else if (walk == 2) k_q8_gemm<EPI, true, 2><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
+    if (walk) return lt_check_launch("k_q8_gemm");
   }
   k_q8_gemm<EPI, kTiled><<<(unsigned)grid, 256, 0, ctx->stream>>>(P);
   return lt_check_launch("k_q8_gemm");
@@ -1267,6 +1279,14 @@ int lt_q8_gemm(lt_ctx* ctx, const void* W, const int8_t* Xq, const uint16_t* Xd,
 int lt_q8_gemm_silu(lt_ctx* ctx, const void* Wgu, const int8_t* Xq, const uint16_t* Xd, float* V, int T, int F,
                     int K) {
   return gemm_silu_entry<false>("lt_q8_gemm_silu", ctx, Wgu, Xq, Xd, V, T, F, K);
+}
+
+int lt_q8_gemm_t_kernel(int num_cus, int T, int N, int K) {
+  if (num_cus <= 0 || T <= 0 || N <= 0 || K <= 0 || K % 32) return -1;
+  GemmParams P{};
+  P.T = T; P.N = N; P.K = K; P.nrt = (N + 31) / 32;
+  const int mode = ls_mode();
+  return mode == 1 || (mode < 0 && take_ls(num_cus, P)) ? 3 : gemm_walk(num_cus, P).walk;
 }
 
 size_t lt_q8_tiles_bytes(int N, int K) {
