@@ -2,7 +2,8 @@
 wrong, against the oracle bit for bit: tiles of 16 query rows and of 16 positions with their
 remainders, chunks of the positions held in LDS (512 and 1024) and one past them, few and many
 tiles, cache values that are not finite in the rows that only part of a tile attends, query rows
-at an odd stride, and splits whose lengths are not multiples of a V block."""
+at an odd stride, and splits whose lengths are not multiples of a V block, of up to 32 positions (a half-wave each in the
+softmax), 33 and 34, 64 to 66 and 87 (a wave each, one and several V blocks)."""
 import ctypes
 
 import numpy as np
@@ -64,7 +65,8 @@ def test_chunk_edges(gpu, oracle, kv_dtype, nh, hd, len0, T):
 
 
 @pytest.mark.parametrize("kv_dtype", [LT_KV_F16, LT_KV_F32])
-@pytest.mark.parametrize("hd,len0,T,nsplit", [(64, 5, 40, 1), (128, 0, 48, 1), (64, 0, 400, 16), (128, 0, 400, 32)])
+@pytest.mark.parametrize("hd,len0,T,nsplit", [(64, 5, 40, 1), (128, 0, 48, 1), (64, 0, 400, 16), (128, 0, 400, 32),
+                                              (64, 300, 400, 16), (128, 700, 400, 16)])
 def test_values_not_finite(gpu, oracle, kv_dtype, hd, len0, T, nsplit):
     """An infinity or a nan in the cache reaches exactly the queries that attend its row."""
     n = len0 + T
@@ -74,7 +76,8 @@ def test_values_not_finite(gpu, oracle, kv_dtype, hd, len0, T, nsplit):
 
 @pytest.mark.parametrize("kv_dtype,hd", [(LT_KV_F16, 64), (LT_KV_F32, 64), (LT_KV_F16, 128), (LT_KV_F32, 128)])
 @pytest.mark.parametrize("len0,T,maxt,nsplit", [(0, 400, 512, 16), (7, 385, 700, 16), (0, 390, 400, 128),
-                                                 (300, 384, 1500, 48)])
+                                                 (300, 384, 1500, 48), (0, 530, 700, 16), (627, 400, 1100, 16),
+                                                 (640, 401, 1041, 16), (1000, 384, 1600, 16)])
 def test_splits(gpu, oracle, kv_dtype, hd, len0, T, maxt, nsplit):
-    rows = sorted({0, 1, 15, 16, 17, 100, 255, 256, 257, T - 18, T - 2, T - 1})
+    rows = sorted({0, 1, 15, 16, 17, 100, 255, 256, 257, T - 18, T - 17, T - 2, T - 1})
     _run(gpu, oracle, kv_dtype, 4, 2, hd, len0, T, maxt, nsplit, rows, T + nsplit, odd_stride=1)
