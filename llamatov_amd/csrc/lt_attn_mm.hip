@@ -91,26 +91,41 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
 
   const uint32_t pitch = (uint32_t)A.nkv * HD * kEb;
   const uint32_t gb = (uint32_t)g * HD * kEb;
-  // (K rows past the tile's last position only make scores that nothing reads, so these loads
-  // need not wait for the length)
-  const __amdgpu_buffer_rsrc_t krsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)A.kc, 0, (int)((uint32_t)A.maxt * pitch), 0x00020000);
-  const __amdgpu_buffer_rsrc_t vrsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)A.vc, 0, (int)((uint32_t)Lmax * pitch), 0x00020000);
+  auto rows_of = [&](const void* c, int rows) {     // the cache's first rows; later rows read zeros
+    return __builtin_amdgcn_make_buffer_rsrc((void*)c, 0, (int)((uint32_t)rows * pitch), 0x00020000);
+  };
 
-  // K tile at position p: unit 4j + g4 of row p + n (rows past the cache read zeros)
+  // loads return in order: the queries first, as B operands (register i of group g4 is q[row n][4i + g4])
+  u32x4 qv[HD / 16];
+  {
+    const int tq = t0 + n < 0 ? 0 : (t0 + n < A.T ? t0 + n : A.T - 1);
+    const float* qs = A.q + (size_t)tq * A.q_stride + (size_t)h * HD;
+#pragma unroll
+    for (int j = 0; j < HD / 16; j++) qv[j] = *(const u32x4_a4*)(qs + 16 * j + 4 * g4);
+  }
+  // K tile at position p: unit 4j + g4 of row p + n.  Only the first waves' first tiles are requested before
+  // the length is known, all else through a descriptor that ends at it
   auto k_off = [&](int p) { return (uint32_t)(p + n) * pitch + gb + (uint32_t)g4 * 16u; };
-  auto load_unit = [&](uint32_t off, int j) {
-    return __builtin_amdgcn_raw_buffer_load_b128(krsrc, (int)(off + 64u * j), 0, 0);
+  auto load_unit = [&](__amdgpu_buffer_rsrc_t k, uint32_t off, int j) {
+    return __builtin_amdgcn_raw_buffer_load_b128(k, (int)(off + 64u * j), 0, 0);
   };
   u32x4 kb[2][NU];                                  // the wave's next two tiles
-  auto load_two = [&](int p) {
+  constexpr int kEarly = 2;
+  if (w < kEarly) {
+    const __amdgpu_buffer_rsrc_t all = rows_of(A.kc, A.maxt);
+#pragma unroll
+    for (int j = 0; j < NU; j++) kb[0][j] = load_unit(all, k_off(w * 16), j);
+  }
+  const __amdgpu_buffer_rsrc_t krsrc = rows_of(A.kc, Lmax), vrsrc = rows_of(A.vc, Lmax);
+  auto load_two = [&](int p, bool first) {
 #pragma unroll
     for (int i = 0; i < 2; i++)
+      if (!first || i == 1 || w >= kEarly) {
 #pragma unroll
-      for (int j = 0; j < NU; j++) kb[i][j] = load_unit(k_off(p + (w + i * NW) * 16), j);
+        for (int j = 0; j < NU; j++) kb[i][j] = load_unit(krsrc, k_off(p + (w + i * NW) * 16), j);
+      }
   };
-  load_two(0);
+  load_two(0, true);
 
   // O: a wave's V dims of RB rows arrive by one 16-byte load per lane and pass through 1 KB of
   // LDS (the wave's own, two blocks in turn) to the lanes: lane (n, g4) feeds dims db + DT n ..
@@ -120,19 +135,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
   const uint32_t vb = gb + (uint32_t)db * kEb + (uint32_t)(l % (SB / 16)) * 16u;
   u32x4 vr[D];
 
-  // the queries as B operands: register i of group g4 is q[row n][4i + g4]
   float qr[HD / 4];
-  {
-    const int tq = t0 + n < 0 ? 0 : (t0 + n < A.T ? t0 + n : A.T - 1);
-    const float* qs = A.q + (size_t)tq * A.q_stride + (size_t)h * HD;
 #pragma unroll
-    for (int j = 0; j < HD / 16; j++) {
-      const u32x4_a4 v = *(const u32x4_a4*)(qs + 16 * j + 4 * g4);
-      uint32_t r[4] = {v.x, v.y, v.z, v.w};
-      transpose4(r);
+  for (int j = 0; j < HD / 16; j++) {
+    uint32_t r[4] = {qv[j].x, qv[j].y, qv[j].z, qv[j].w};
+    transpose4(r);
 #pragma unroll
-      for (int e = 0; e < 4; e++) qr[4 * j + e] = __uint_as_float(r[e]);
-    }
+    for (int e = 0; e < 4; e++) qr[4 * j + e] = __uint_as_float(r[e]);
   }
   // a tile's scores: register r of (row n, group g4) is position 4 g4 + r; each unit is
   // replaced by that of the tile two ahead as soon as it is taken
@@ -149,7 +158,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
                          __builtin_amdgcn_perm(k.z, k.x, 0x07060302u),
                          __builtin_amdgcn_perm(k.w, k.y, 0x05040100u),
                          __builtin_amdgcn_perm(k.w, k.y, 0x07060302u)};
-        kt[j] = load_unit(next, j);
+        kt[j] = load_unit(krsrc, next, j);
         transpose4(r);
 #pragma unroll
         for (int s = 0; s < 4; s++) {
@@ -158,7 +167,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
         }
       } else {
         uint32_t r[4] = {k.x, k.y, k.z, k.w};
-        kt[j] = load_unit(next, j);
+        kt[j] = load_unit(krsrc, next, j);
         transpose4(r);
 #pragma unroll
         for (int s = 0; s < 4; s++) acc = mma(__uint_as_float(r[s]), qr[4 * j + s], acc);
@@ -242,7 +251,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
     // the maxima: with the scores where they all fit, in a pass of their own else
     if (multi) {
       score(0, Lmax, false, true);
-      load_two(0);
+      load_two(0, false);
     } else {
       score(0, Lmax, true, true);
     }
@@ -320,7 +329,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 3)))
         }
       }
       if (multi) {
-        load_two(c1);
+        load_two(c1, false);
         __syncthreads();                            // the next chunk rewrites P
       }
     }
