@@ -438,6 +438,11 @@ LT_API int lt_len_add_n(lt_ctx* ctx, int* len, int n, int T, int maxt);
 LT_API int lt_attn_prefill(lt_ctx* ctx, const float* q, int q_stride, const void* kc, const void* vc,
                            const int* len0, float* out, int T, int nh, int nkv, int hd, float scale, int maxt,
                            int nsplit, int kv_dtype, void* ws, size_t ws_bytes);
+/* lt_attn_prefill told on the host where the context ends: end = *len0 + T (0: not known).  It decides between
+ * kernels of equal results and nothing else. */
+LT_API int lt_attn_prefill_end(lt_ctx* ctx, const float* q, int q_stride, const void* kc, const void* vc,
+                               const int* len0, float* out, int T, int nh, int nkv, int hd, float scale, int maxt,
+                               int nsplit, int kv_dtype, void* ws, size_t ws_bytes, int end);
 
 /* Embedding rows of T device token ids (lt_embed_q8 per token), x [T][E]. */
 LT_API int lt_embed_q8_batch(lt_ctx* ctx, const void* emb, const int* toks, float* x, int T, int E, int vocab,

@@ -121,6 +121,8 @@ _SIGS = {
     "lt_len_add_n": (c_int, [_P, _P, c_int, c_int, c_int]),
     "lt_attn_prefill": (c_int, [_P, _P, c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_int,
                                 c_int, c_int, _P, c_size_t]),
+    "lt_attn_prefill_end": (c_int, [_P, _P, c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_int,
+                                    c_int, c_int, _P, c_size_t, c_int]),
     "lt_embed_q8_batch": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, _P]),
     "lt_selftest_numerics": (c_int, [_P, _P]),
     "lt_selftest_attn_numerics": (c_int, [_P, _P]),

@@ -1570,9 +1570,9 @@ bool use_w1() {
 }
 
 // Launches the attention (and the merge when nsplit > 1) for `rows` query rows with hpw
-// heads per workgroup.
+// heads per workgroup.  end: the context's length as far as the caller knows it, for the choice of a kernel.
 int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, void* ws, size_t ws_bytes,
-                const char* what) {
+                const char* what, int end = 0) {
   LT_REQUIRE(A.nsplit <= 128, "%s: nsplit=%d (at most 128)", what, A.nsplit);
   // the single-wave kernel (every mode): all heads of a KV group share its K/V reads
   const int rep = A.nh / A.nkv;
@@ -1619,7 +1619,8 @@ int launch_attn(lt_ctx* ctx, int mode, bool f16, int hpw, int rows, AttnArgs A, 
                   (f16 ? (dpl == 1 || dpl == 2 || dpl == 4) : (dpl == 1 || dpl == 2)) && w1_shm <= 64 * 1024;
   // prefill on the matrix cores, for what the per-row kernels take too (their LDS limits and the
   // workspace the caller owes a split context stand)
-  const bool mm = mode == AM_PREFILL && use_mm() && lt_attn_mm_covers(A.hd, rows, A.maxt, A.nsplit) &&
+  const int known = w1 && end > 0 && end < A.maxt ? end : A.maxt;
+  const bool mm = mode == AM_PREFILL && use_mm() && lt_attn_mm_covers(A.hd, f16, rows, A.maxt, known, A.nsplit) &&
                   (w1 || ((size_t)hpw * A.hd + 2 * A.hd + (size_t)hpw * per_max + kVChunkFloats) * sizeof(float) <=
                              64 * 1024);
   auto launch_mm = [&]() {
@@ -1932,9 +1933,9 @@ int lt_attn_decode_noalloc(lt_ctx* ctx, const float* q, const void* kc, const vo
                      ctx->attn_scratch, ctx->attn_scratch_bytes, "lt_attn_decode_noalloc");
 }
 
-int lt_attn_prefill(lt_ctx* ctx, const float* q, int q_stride, const void* kc, const void* vc, const int* len0,
-                    float* out, int T, int nh, int nkv, int hd, float scale, int maxt, int nsplit, int kv_dtype,
-                    void* ws, size_t ws_bytes) {
+int lt_attn_prefill_end(lt_ctx* ctx, const float* q, int q_stride, const void* kc, const void* vc, const int* len0,
+                        float* out, int T, int nh, int nkv, int hd, float scale, int maxt, int nsplit, int kv_dtype,
+                        void* ws, size_t ws_bytes, int end) {
   LT_REQUIRE(ctx && q && kc && vc && len0 && out, "lt_attn_prefill: null argument");
   LT_REQUIRE(T > 0 && q_stride >= nh * hd, "lt_attn_prefill: T=%d q_stride=%d", T, q_stride);
   const size_t cb = cache_bytes_of(1, maxt, nkv, hd, kv_dtype);
@@ -1945,7 +1946,14 @@ int lt_attn_prefill(lt_ctx* ctx, const float* q, int q_stride, const void* kc, c
   // the T query rows of one sequence re-read the same rows: the heads of a KV group share
   // each workgroup whenever the group divides
   return launch_attn(ctx, AM_PREFILL, kv_dtype == LT_KV_F16, pick_hpw(nh, nkv, hd, (size_t)1 << 30), T, A, ws,
-                     ws_bytes, "lt_attn_prefill");
+                     ws_bytes, "lt_attn_prefill", end);
+}
+
+int lt_attn_prefill(lt_ctx* ctx, const float* q, int q_stride, const void* kc, const void* vc, const int* len0,
+                    float* out, int T, int nh, int nkv, int hd, float scale, int maxt, int nsplit, int kv_dtype,
+                    void* ws, size_t ws_bytes) {
+  return lt_attn_prefill_end(ctx, q, q_stride, kc, vc, len0, out, T, nh, nkv, hd, scale, maxt, nsplit, kv_dtype, ws,
+                             ws_bytes, 0);
 }
 
 int lt_attn_step(lt_ctx* ctx, const float* qkv, const float* freqs, void* kc, void* vc, const int* len,

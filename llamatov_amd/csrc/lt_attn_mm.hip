@@ -518,13 +518,18 @@ size_t mm_lds(int cap, int nsplit) {
 
 // Splits cost a merge of the chains per split and tile whatever the length, so short prompts
 // stay on the per-row kernel (16 splits, 32 heads of 128, maxt 1024, per-row / here: T = 100
-// 19.0 / 22.3 us, 200 28.7 / 42.3, 512 106 / 95, and at maxt 512 87 / 71).  So do caches of at most
-// 32 rows of 128: one score tile or two leave most waves idle (32 heads, T = 16 and 32, fp16 7.3 /
-// 8.0 and 7.4 / 8.1, fp32 6.7 / 8.2 and 7.2 / 8.7; at 48 rows 9.5 / 8.7 and 9.6 / 9.1; heads of 64
-// are even from T = 8 on).
-bool lt_attn_mm_covers(int hd, int T, int maxt, int nsplit) {
+// 19.0 / 22.3 us, 200 28.7 / 42.3, 512 106 / 95, and at maxt 512 87 / 71).  So do the shortest contexts, a
+// tile or a few of which leave most waves idle, where the caller knows them (us over caches of 1024 rows):
+//   T at 0 cached       16          32          48          64          100         135
+//   14 of 64, fp16      3.9 / 5.4   4.0 / 5.5   4.6 / 5.9   4.7 / 6.0   6.9 / 7.2   9.8 / 8.8
+//   14 of 64, fp32      4.0 / 5.5   4.1 / 5.7   4.9 / 6.0   5.0 / 6.3   8.2 / 7.2   13.3 / 8.9
+//   32 of 128, fp16     5.9 / 7.3   6.0 / 7.3   8.0 / 8.0   8.2 / 8.2   13.0 / 10.1 24.2 / 12.9
+//   32 of 128, fp32     5.3 / 7.5   5.8 / 7.7   8.0 / 8.2   8.8 / 8.8   14.2 / 10.4 25.3 / 13.6
+// (16 at 100 cached: 6.0 / 7.7, 6.8 / 7.7, 12.1 / 10.3, 13.1 / 10.9; at 500: 17.2 / 16.3, 19.1 / 16.1,
+// 40.5 / 23.1, 44.9 / 23.2).
+bool lt_attn_mm_covers(int hd, bool f16, int T, int maxt, int end, int nsplit) {
   if (hd != 64 && hd != 128) return false;
-  if (nsplit == 1) return hd == 64 || maxt > 32;
+  if (nsplit == 1) return end > (hd == 128 ? 32 : f16 ? 112 : 64);
   return (nsplit % 16 == 0 && T >= 384 && mm_lds((maxt + 63) & ~63, nsplit) <= (size_t)kLds);
 }
 

@@ -81,9 +81,9 @@ struct LtAttnMm {
   int maxt, nsplit;
   int cap, ntiles;   // set by the launcher: positions held in LDS, 16-row tiles in the grid
 };
-// Head sizes 64 and 128; one split, or a multiple of 16 splits over a long prompt whose context
-// fits in LDS.
-bool lt_attn_mm_covers(int hd, int T, int maxt, int nsplit);
+// Head sizes 64 and 128; one split past the shortest contexts (end: the most positions a row attends, as
+// far as the caller knows), or a multiple of 16 splits over a long prompt whose context fits in LDS.
+bool lt_attn_mm_covers(int hd, bool f16, int T, int maxt, int end, int nsplit);
 int lt_attn_mm_prefill(lt_ctx* ctx, LtAttnMm A, int hd, bool f16);
 
 // Unsplit decode attention, one workgroup per (head, sequence) (lt_attn_head.hip): the decode

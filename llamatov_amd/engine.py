@@ -1265,7 +1265,7 @@ def forward_prefill(plan: DecodePlan, tokens, embeddings: np.ndarray | None = No
         D.h2d(B.toks.ptr, toks)
         call("lt_embed_q8_batch", h, m.tok_embd.t.vp, B.toks.vp, B.x.vp, T, E, cfg.vocab, plan.err.vp)
     _prefill_layers(m, p, B, T, [(c.k.vp, c.v.vp, _vp(c.len_ptr)) for c in plan.caches], plan.max_ctx,
-                    plan.scale)
+                    plan.caches[0].length + T, plan.scale)
     call("lt_len_add_n", h, _vp(plan.lens.ptr), len(m.layers), T, plan.max_ctx)
     for cache in plan.caches:   # the host mirror advances with the device lengths
         cache.length += T
@@ -1285,9 +1285,10 @@ SILU_QUANT_MAX_T = 512
 
 
 def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, caches: list, maxt: int,
-                    scale: float) -> None:
+                    end: int, scale: float) -> None:
     """The layers of a batched prefill of the T rows in B.x, one sequence: caches[il] =
-    (k, v, len) device pointers of layer il's cache and its length (read, not advanced)."""
+    (k, v, len) device pointers of layer il's cache and its length (read, not advanced), end the
+    context's length with the T rows (for the choice of the attention kernel)."""
     cfg, h = m.cfg, m.dev.handle
     E, F, hd, nh, nkv = cfg.n_embd, cfg.n_ff, cfg.head_dim, cfg.n_head, cfg.n_head_kv
     QD, NQ = cfg.q_dim, cfg.n_qkv
@@ -1298,8 +1299,8 @@ def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, cac
         call("lt_rmsnorm_quant_bm", h, B.x.vp, L["attn_norm"].vp, B.xq.vp, B.xd.vp, T, E, eps)
         call("lt_q8_gemm_t", h, L["wqkv_t"].t.vp, B.xq.vp, B.xd.vp, _vp(L["bqkv"]), None, B.qkv.vp, T, NQ, E)
         call("lt_rope_append_batch", h, B.qkv.vp, T, NQ, lp, nh, nkv, hd, m.freqs.vp, kp, vp, maxt, p.kv_dtype)
-        call("lt_attn_prefill", h, B.qkv.vp, NQ, kp, vp, lp, B.att.vp, T, nh, nkv, hd, ctypes.c_float(scale), maxt,
-             p.attn_nsplit, p.kv_dtype, ws, ws_n)
+        call("lt_attn_prefill_end", h, B.qkv.vp, NQ, kp, vp, lp, B.att.vp, T, nh, nkv, hd, ctypes.c_float(scale), maxt,
+             p.attn_nsplit, p.kv_dtype, ws, ws_n, end)
         call("lt_quant_q8_bm", h, B.att.vp, B.xq.vp, B.xd.vp, T, QD)
         call("lt_q8_gemm_t", h, L["wo_t"].t.vp, B.xq.vp, B.xd.vp, None, B.x.vp, B.xres.vp, T, E, QD)
         call("lt_rmsnorm_quant_bm", h, B.xres.vp, L["ffn_norm"].vp, B.xq.vp, B.xd.vp, T, E, eps)
@@ -1637,7 +1638,8 @@ class BatchDecodePlan:
         lp = self.lens.ptr + 4 * b
         off = b * self.slot_bytes
         _prefill_layers(m, self.profile, Bf, T, [(self.k[il].ptr + off, self.v[il].ptr + off, lp)
-                                                 for il in range(cfg.n_layers)], self.max_ctx, self.scale)
+                                                 for il in range(cfg.n_layers)], self.max_ctx,
+                        self.length[b] + T, self.scale)
         call("lt_len_add", h, _vp(lp), T, self.max_ctx)
         call("lt_len_add", h, _vp(self.lens.ptr + 4 * (self.B + b)), T, self.max_ctx)
         self.length[b] += T

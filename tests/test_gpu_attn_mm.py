@@ -16,10 +16,10 @@ from llamatov_amd._lib import LT_KV_F16, LT_KV_F32, call
 pytestmark = pytest.mark.gpu
 
 
-def _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, maxt, nsplit, rows, seed, odd_stride=0, bad=()):
+def _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, maxt, nsplit, rows, seed, odd_stride=0, bad=(), end=0):
     f16 = kv_dtype == LT_KV_F16
     print(f"[gpu-case] attn mm nh={nh} nkv={nkv} hd={hd} f16={f16} len0={len0} T={T} maxt={maxt} "
-          f"nsplit={nsplit} bad={bad}", flush=True)
+          f"nsplit={nsplit} bad={bad} end={end}", flush=True)
     rng = np.random.default_rng(seed)
     stride = nh * hd + odd_stride
     q = rng.standard_normal((T, stride)).astype(np.float32)
@@ -36,8 +36,8 @@ def _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, maxt, nsplit, rows, seed, 
     out = dr.DevTensor.empty((T, nh * hd), np.float32, gpu)
     scale = float(hd ** -0.5)
     ts = [up(q), up(kd), up(vd), up(np.array([len0], np.int32))]
-    call("lt_attn_prefill", gpu.handle, ts[0].vp, stride, ts[1].vp, ts[2].vp, ts[3].vp, out.vp, T, nh, nkv, hd,
-         ctypes.c_float(scale), maxt, nsplit, kv_dtype, ws.vp, ws.nbytes)
+    call("lt_attn_prefill_end", gpu.handle, ts[0].vp, stride, ts[1].vp, ts[2].vp, ts[3].vp, out.vp, T, nh, nkv, hd,
+         ctypes.c_float(scale), maxt, nsplit, kv_dtype, ws.vp, ws.nbytes, end)
     got = out.to_host()
     for t in rows:
         exp = oracle.attn_decode(np.ascontiguousarray(q[t, : nh * hd]), kd, vd, len0 + t + 1, nh, nkv, hd, scale, f16,
@@ -53,6 +53,17 @@ def _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, maxt, nsplit, rows, seed, 
 @pytest.mark.parametrize("len0,T", [(0, 1), (0, 15), (0, 16), (0, 17), (3, 65), (31, 33), (49, 64)])
 def test_tile_edges(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T):
     _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, len0 + T + 3, 1, range(T), 5 * T + len0, odd_stride=3)
+
+
+@pytest.mark.parametrize("kv_dtype", [LT_KV_F16, LT_KV_F32])
+@pytest.mark.parametrize("nh,nkv,hd", [(14, 2, 64), (4, 1, 128)])
+@pytest.mark.parametrize("len0,T", [(0, 32), (1, 32), (40, 24), (41, 24), (0, 112), (96, 17), (0, 200)])
+@pytest.mark.parametrize("end", [0, None, 1, 1 << 30])
+def test_context_end(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, end):
+    """The known end of the context, at both sides of each line it draws, unknown and wrong."""
+    rows = sorted({0, 1, 15, 16, T - 17, T - 1})
+    _run(gpu, oracle, kv_dtype, nh, nkv, hd, len0, T, 400, 1, rows, T + len0, odd_stride=1,
+         end=len0 + T if end is None else end)
 
 
 # (few workgroups: 8 waves and chunks of 1024; more than one per CU: 4 waves and chunks of 512)
