@@ -1193,6 +1193,20 @@ class DecodePlan:
                 t.free()
 
 
+# up to this width and this many tokens a prefill's gate|up launch also quantizes its SiLU output
+# (lt_q8_gemm_silu_quant_t), which spares a launch and the fp32 round trip; wider, the kernel that
+# walks K in one go per row tile loses more than that.  Cold weights, two launches / one (us): 9728 x
+# 896 at T = 16 8.2 / 6.4, 64 9.9 / 9.2, 256 19.0 / 17.2, 509 30.6 / 30.3; 28672 x 4096 at T = 8 30.9
+# / 31.0, 64 46.8 / 58.1, 512 210 / 347
+SILU_QUANT_MAX_EMBD = 1024
+SILU_QUANT_MAX_T = 512
+
+
+def silu_quant_rows(cfg) -> int:
+    """The longest prompt whose gate|up launch also quantizes (0: none does)."""
+    return SILU_QUANT_MAX_T if cfg.n_embd <= SILU_QUANT_MAX_EMBD and cfg.n_ff % 32 == 0 else 0
+
+
 class PrefillBuffers:
     """Device buffers of a batched prefill of up to T tokens."""
 
@@ -1209,8 +1223,9 @@ class PrefillBuffers:
         self.v = DevTensor.empty((T, F), np.float32, D)
         self.xq = DevTensor.empty((T * kmax,), np.int8, D)
         self.xd = DevTensor.empty((T * kmax // 32,), np.uint16, D)
-        self.vq = DevTensor.empty((T * F,), np.int8, D)
-        self.vd = DevTensor.empty((T * F // 32,), np.uint16, D)
+        n = min(T, silu_quant_rows(cfg)) * F
+        self.vq = DevTensor.empty((n,), np.int8, D) if n else None
+        self.vd = DevTensor.empty((n // 32,), np.uint16, D) if n else None
         aw = _lib.raw("lt_attn_workspace_size")(T, cfg.n_head, cfg.head_dim, plan.profile.attn_nsplit)
         self.ws = DevTensor.empty((aw,), np.uint8, D) if aw else None
 
@@ -1275,15 +1290,6 @@ def forward_prefill(plan: DecodePlan, tokens, embeddings: np.ndarray | None = No
          cfg.vocab, E, plan.tok.vp, None, None, 0, plan.am_ws.vp, plan.am_ws.nbytes)
 
 
-# up to this width and this many tokens a prefill's gate|up launch also quantizes its SiLU output
-# (lt_q8_gemm_silu_quant_t), which spares a launch and the fp32 round trip; wider, the kernel that
-# walks K in one go per row tile loses more than that.  Cold weights, two launches / one (us): 9728 x
-# 896 at T = 16 8.2 / 6.4, 64 9.9 / 9.2, 256 19.0 / 17.2, 509 30.6 / 30.3; 28672 x 4096 at T = 8 30.9
-# / 31.0, 64 46.8 / 58.1, 512 210 / 347
-SILU_QUANT_MAX_EMBD = 1024
-SILU_QUANT_MAX_T = 512
-
-
 def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, caches: list, maxt: int,
                     end: int, scale: float) -> None:
     """The layers of a batched prefill of the T rows in B.x, one sequence: caches[il] =
@@ -1304,7 +1310,7 @@ def _prefill_layers(m: ResidentModel, p: Profile, B: PrefillBuffers, T: int, cac
         call("lt_quant_q8_bm", h, B.att.vp, B.xq.vp, B.xd.vp, T, QD)
         call("lt_q8_gemm_t", h, L["wo_t"].t.vp, B.xq.vp, B.xd.vp, None, B.x.vp, B.xres.vp, T, E, QD)
         call("lt_rmsnorm_quant_bm", h, B.xres.vp, L["ffn_norm"].vp, B.xq.vp, B.xd.vp, T, E, eps)
-        if E <= SILU_QUANT_MAX_EMBD and T <= SILU_QUANT_MAX_T and F % 32 == 0:
+        if T <= silu_quant_rows(cfg):
             call("lt_q8_gemm_silu_quant_t", h, L["wgu_il_t"].t.vp, B.xq.vp, B.xd.vp, B.vq.vp, B.vd.vp, T, F, E)
             vq, vd = B.vq.vp, B.vd.vp
         else:

@@ -145,3 +145,18 @@ def test_resident_cache_keys_on_the_dict_and_its_content(monkeypatch):
     dr.release_resident(w1)
     dr.release_resident(w2)
     assert m1b.freed and m2.freed and not dr._MODELS
+
+
+@pytest.mark.parametrize("n_embd,n_ff,T,rows", [(1024, 4864, 8, 8), (896, 4864, 512, 512), (896, 4864, 8192, 512),
+                                                (1056, 4864, 512, 0), (4096, 14336, 8192, 0), (896, 80, 64, 0)])
+def test_prefill_buffers_hold_only_what_is_launched(monkeypatch, n_embd, n_ff, T, rows):
+    """The quantized SiLU output has room for the prompts whose gate|up launch writes it and no more."""
+    from types import SimpleNamespace
+    from llamatov_amd import engine
+    monkeypatch.setattr(engine.DevTensor, "empty",
+                        lambda shape, dtype, dev: SimpleNamespace(shape=shape, free=lambda: None))
+    cfg = SimpleNamespace(n_embd=n_embd, n_ff=n_ff, q_dim=n_embd, n_qkv=n_embd, n_head=2, head_dim=64)
+    B = engine.PrefillBuffers(SimpleNamespace(cfg=cfg, dev=None, profile=SimpleNamespace(attn_nsplit=1)), T)
+    assert min(T, engine.silu_quant_rows(cfg)) == rows
+    assert [t and t.shape for t in (B.vq, B.vd)] == ([(rows * n_ff,), (rows * n_ff // 32,)] if rows else [None, None])
+    B.free()
