@@ -208,7 +208,7 @@ def step_kernels(dev, plan, only: str | None = None, attn_len: int | None = None
                     bytes=rb(NQ, E) + 8 * E + 8 * NQ,
                     fn=lambda w, il: call("lt_q8_gemv_rms", h, plan.carry.vp, m.layers[il]["attn_norm"].vp, eps,
                                           w.vp, dr._vp(m.layers[il]["bqkv"]), plan.qkv.vp, NQ, E)),
-        "attn": dict(kernel="k_attn_w1<f16, STEP> (lt_attn_step)", shape=[nh, nkv, hd, L + 1],
+        "attn": dict(kernel="k_attn_head<f16, STEP> (lt_attn_step)", shape=[nh, nkv, hd, L + 1],
                      mats=None, count=cfg.n_layers,
                      bytes=2 * (L + 1) * cfg.kv_dim * 2 + 4 * NQ + QD + QD // 16,
                      fn=lambda w, il: call("lt_attn_step", h, plan.qkv.vp, m.freqs.vp, plan.caches[il].k.vp,
@@ -454,9 +454,9 @@ def c5_leg(dev, n_prefill: int = 512, n_decode: int = 256, eager: bool = False, 
     plan = dr.DecodePlan(model, dr.Profile(kv_dtype=LT_KV_F16, attn_nsplit=C5_ATTN_NSPLIT),
                          max_ctx=n_prefill + n_decode + 8, hist_cap=4096)
     prompt = M.random_prompt(cfg, n_prefill, seed=17)
-    # warm the prefill kernels on a short prompt, then rewind
-    dr.forward_prefill(plan, prompt[:8])
-    plan.prefill_buffers(n_prefill)      # activation buffers are set-up, not prefill work
+    # warm the prefill's kernels, which depend on the prompt's length (a kernel's first launch loads its code,
+    # about 1 ms), and its activation buffers; then rewind
+    dr.forward_prefill(plan, prompt)
     dev.sync()
     plan.reset()
     ev = Events(dev)
