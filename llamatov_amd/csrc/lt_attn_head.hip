@@ -1,6 +1,7 @@
 // lt_attn_head.hip -- decode attention of one query head over one sequence's cache, unsplit (the
 // single-pass order of k_attn_decode_masked): the decode step (RoPE, KV append, attention,
-// quant) and batched decode, bit-identical to k_attn_w1 and k_attn_dec of lt_attn.hip.
+// quant) and batched decode, bit-identical to k_attn_w1 and k_attn_dec of lt_attn.hip (but for the sign
+// of a zero that underflowed products left: lt_attn_mm.hip).
 //
 // The unsplit order leaves one serial chain per (head, dim) over all positions, so a head's
 // latency is what counts: a workgroup of NW waves takes one head and shares out everything that

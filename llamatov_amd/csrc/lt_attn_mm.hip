@@ -5,7 +5,8 @@
 // ascending k, each with one rounding: the sequential fma chain of the reference's scores
 // (over the dims) and of its outputs (over the positions), for 16 x 16 chains at once.
 // Checked on the device against fmaf chains of 512 terms over normal, subnormal and
-// wide-range operands (all bits equal); the parity tests compare whole results.
+// wide-range operands, zeros, infinities and nans (lt_selftest_attn_numerics: all bits equal);
+// the parity tests compare whole results.
 //
 // One workgroup takes 16 consecutive query rows of one head, aligned to a cache position that
 // is a multiple of 16, and its NW waves share the work:
@@ -23,7 +24,9 @@
 // fold's partial sums and the output chains carried over.
 //
 // Rows of one tile attend up to 15 positions more or less; a masked exp is 0 and
-// fma(0, v, o) = o for every finite v.  Where V is not finite in the rows that only part of
+// fma(0, v, o) = o for every finite v and every o but -0, which becomes +0.  (A chain that
+// starts at +0 reaches -0 only where its products all underflow: there a zero's sign may differ
+// from the per-row kernels'.)  Where V is not finite in the rows that only part of
 // the tile attends, those steps run one position at a time with a select instead.
 //
 // Bound: the vector units' issue.  An fp32 matrix instruction holds its SIMD for 32 cycles (1024
@@ -31,8 +34,8 @@
 // before every one: 52 cycles a pair), so the conversions of fp16 rows, the transposes and the
 // binary64 exps add to the matrix time.  Measured against the per-row kernel (k_attn_w1): T =
 // 2048, 32 heads of 128 over 8 KV heads, fp16, one split: 1772 -> 572 us (60 TF of the 157 TF
-// fp32 matrix peak; a third of its score work is the second pass); T = 512: 97 -> 39.6 us;
-// T = 509, 14 heads of 64: 41.7 -> 18.5 us.
+// fp32 matrix peak; the second pass is 48% of its score work, a third of scores and outputs
+// together); T = 512: 97 -> 39.6 us; T = 509, 14 heads of 64: 41.7 -> 18.5 us.
 #include "lt_q8_device.h"
 
 namespace {
