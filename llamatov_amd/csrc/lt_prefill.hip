@@ -1128,7 +1128,8 @@ GemmWalk gemm_walk(long cus, const GemmParams& P) {
 //  - two, not in groups: below 10: 8960 x 1536 at 128 (4.4) / 768 (26, three rounds) / 1024 (35) 26.6 / 18.1,
 //    78 / 75, 91.4 / 98.1; 1536 x 1536 at 1024 (6) / 2048 (12) 25.3 / 17.6, 32.7 / 35.1;
 //  - three to five: up to 128 tokens, and below 7 on the 4-slot walk, 9 on the dynamic walk of at most four, else
-//    8: 28672 x 4096 at 64 / 128 71.7 / 47.1, 78.5 / 76.7, 160 (18, three rounds) 126 / 90, 256 (28) 130 / 135;
+//    8: 28672 x 4096 at 64 / 128 71.7 / 47.1, 78.5 / 76.7 (with the SiLU epilogue 72.9 / 74.5, which the line
+//    at 128 leaves there), 160 (18, three rounds) 126 / 90, 256 (28) 130 / 135;
 //    4096 x 4096 at 400 (6.5) 35.0 / 34.4, 512 (8) 36.1 / 40.1; 6144 x 4096 at 320 (7.5) 43.7 / 38.4, 400 (9.8)
 //    44.7 / 47.9; 896 x 4864 at 512 (2) / 2048 (8) 41.8 / 14.7, 47.7 / 51.2; 3584 x 3584 at 640 (8.75) 48.2 /
 //    39.2, 672 (9) 48.2 / 40.2, 1024 (14, two rounds) 75 / 64, but 18944 x 3584 at 256 (18.5, two) 87.6 / 89.1
